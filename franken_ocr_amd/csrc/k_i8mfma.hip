@@ -45,6 +45,7 @@
 // 1 KB contiguous. Read in the upload layout ([E][N][K], output-channel-major,
 // what decode uses), each load touched 32 rows — 32 cache lines — and the
 // L1 address path, not the MFMA, bound the kernel (TA busy 74%, MFMA 12%).
+#include <algorithm>
 #include <type_traits>
 
 #include "focr_internal.hpp"
@@ -62,14 +63,16 @@ constexpr int KC = 256;               // K bytes per staged activation chunk
 constexpr int PPR = KC / 16;          // 16-byte pieces per staged row (a multiple of 16: the swizzle)
 constexpr int SPC = KC / KB;          // stages per chunk
 constexpr int kXcds = 8;
-constexpr int kRing = 2;              // K stages of weight fragments in flight
+constexpr int kRingTiles = 4;         // weight fragments in flight per wave: K stages x column tiles
 static_assert(PPR % 16 == 0, "the LDS swizzle permutes pieces within groups of 16");
 
 enum I8Epi { kI8Linear = 0, kI8Swiglu = 1, kI8Down = 2 };
 
-template <int EPI>
+// Columns per block: NJ column tiles of 32 per wave (for SwiGLU one of the
+// gate and one of the up matrix).
+template <int EPI, int NJ = 2>
 constexpr int bcols() {
-    return EPI == kI8Swiglu ? 128 : 256;
+    return EPI == kI8Swiglu ? 128 : 128 * NJ;
 }
 
 struct I8Args {
@@ -89,7 +92,7 @@ struct I8Args {
 
 // One block tile: rows [r0, r0 + nr) (nr <= 64) of expert e against column
 // block cb. Every thread of the block calls it (it synchronises).
-template <int EPI>
+template <int EPI, int NJ = 2>
 __device__ __forceinline__ void i8_tile(const I8Args& a, int e, int r0, int nr, int cb) {
     // two chunk buffers
     __shared__ __align__(16) int8_t lds_a0[BM * KC];
@@ -105,6 +108,7 @@ __device__ __forceinline__ void i8_tile(const I8Args& a, int e, int r0, int nr, 
     const int c32 = l & 31;
     const int K = a.K, N = a.N;
     const int S = K / KB;
+    constexpr int kRing = kRingTiles / NJ;
 
     if (tid < BM) {
         const int row = r0 + (tid < nr ? tid : nr - 1);  // rows past nr repeat the last one, never stored
@@ -125,27 +129,27 @@ __device__ __forceinline__ void i8_tile(const I8Args& a, int e, int r0, int nr, 
     // this lane's two weight columns (tile j = 0, 1) and their fragment
     // streams: 1 KB per (column tile, 32-byte K step), lane l at 16 l
     const int NT = (N + 31) >> 5, KS = K >> 5;
-    int col[2];
-    const int8_t* bp[2];
+    int col[NJ];
+    const int8_t* bp[NJ];
 #pragma unroll
-    for (int j = 0; j < 2; ++j) {
-        const int tile = EPI == kI8Swiglu ? cb * 4 + wave : cb * 8 + 2 * wave + j;
+    for (int j = 0; j < NJ; ++j) {
+        const int tile = EPI == kI8Swiglu ? cb * 4 + wave : NJ * (cb * 4 + wave) + j;
         col[j] = 32 * tile + c32;
         const int8_t* B = (EPI == kI8Swiglu && j == 1) ? a.B1 : a.B0;
         bp[j] = B + (static_cast<size_t>(e * NT + (tile < NT ? tile : NT - 1)) * KS * 64 + l) * 16;
     }
     // fragments f[2 j + s]: column tile j, K step s of stage st (clamped past the end)
-    auto load_b = [&](int st, v4i (&f)[4]) {
+    auto load_b = [&](int st, v4i (&f)[2 * NJ]) {
         const int ss = st < S ? st : S - 1;
 #pragma unroll
-        for (int j = 0; j < 2; ++j)
+        for (int j = 0; j < NJ; ++j)
 #pragma unroll
             for (int s = 0; s < 2; ++s)
                 f[2 * j + s] = *reinterpret_cast<const v4i*>(bp[j] + static_cast<size_t>(2 * ss + s) * 1024);
     };
     // a ring of kRing stages of fragments, stage st in f[st % kRing], loaded
     // kRing stages ahead (SPC a multiple of kRing keeps the ring index a constant)
-    v4i f[kRing][4];
+    v4i f[kRing][2 * NJ];
 #pragma unroll
     for (int q = 0; q < kRing; ++q) load_b(q, f[q]);
     __syncthreads();  // the row tables
@@ -180,7 +184,7 @@ __device__ __forceinline__ void i8_tile(const I8Args& a, int e, int r0, int nr, 
     // live = false (a stage past K): the weight fragments are zeroed by a
     // select, so the MFMAs add nothing and the code stays branch-free (a
     // branch around them costs the compiler its exact load-count waits).
-    auto compute = [&](const int8_t* buf, int ls, const v4i (&f)[4], bool live) {
+    auto compute = [&](const int8_t* buf, int ls, const v4i (&f)[2 * NJ], bool live) {
         const v4i z = {0, 0, 0, 0};
 #pragma unroll
         for (int s = 0; s < 2; ++s) {
@@ -188,11 +192,13 @@ __device__ __forceinline__ void i8_tile(const I8Args& a, int e, int r0, int nr, 
             const v4i a0 = *reinterpret_cast<const v4i*>(buf + c32 * KC + 16 * (c16 ^ (c32 & 15)));
             const v4i a1 = *reinterpret_cast<const v4i*>(buf + (32 + c32) * KC + 16 * (c16 ^ ((32 + c32) & 15)));
             const v4i b0 = live ? f[s] : z;
-            const v4i b1 = live ? f[2 + s] : z;
             acc00 = __builtin_amdgcn_mfma_i32_32x32x32_i8(a0, b0, acc00, 0, 0, 0);
-            acc01 = __builtin_amdgcn_mfma_i32_32x32x32_i8(a0, b1, acc01, 0, 0, 0);
             acc10 = __builtin_amdgcn_mfma_i32_32x32x32_i8(a1, b0, acc10, 0, 0, 0);
-            acc11 = __builtin_amdgcn_mfma_i32_32x32x32_i8(a1, b1, acc11, 0, 0, 0);
+            if constexpr (NJ == 2) {
+                const v4i b1 = live ? f[2 + s] : z;
+                acc01 = __builtin_amdgcn_mfma_i32_32x32x32_i8(a0, b1, acc01, 0, 0, 0);
+                acc11 = __builtin_amdgcn_mfma_i32_32x32x32_i8(a1, b1, acc11, 0, 0, 0);
+            }
         }
     };
 
@@ -224,12 +230,13 @@ __device__ __forceinline__ void i8_tile(const I8Args& a, int e, int r0, int nr, 
     }
 
     // epilogue
-    const bool ok0 = col[0] < N, ok1 = col[1] < N;
+    const int col1 = NJ == 2 ? col[NJ - 1] : N;  // one column tile: no second column
+    const bool ok0 = col[0] < N, ok1 = col1 < N;
     const float ws0 = a.s0[static_cast<size_t>(e) * N + (ok0 ? col[0] : 0)];
     const float ws1 = EPI == kI8Swiglu ? a.s1[static_cast<size_t>(e) * N + (ok0 ? col[0] : 0)]
-                                       : a.s0[static_cast<size_t>(e) * N + (ok1 ? col[1] : 0)];
+                                       : a.s0[static_cast<size_t>(e) * N + (ok1 ? col1 : 0)];
     const float b0 = (EPI == kI8Linear && a.bias) ? a.bias[ok0 ? col[0] : 0] : 0.0f;
-    const float b1 = (EPI == kI8Linear && a.bias) ? a.bias[ok1 ? col[1] : 0] : 0.0f;
+    const float b1 = (EPI == kI8Linear && a.bias) ? a.bias[ok1 ? col1 : 0] : 0.0f;
 #pragma unroll
     for (int t = 0; t < 2; ++t) {
 #pragma unroll
@@ -256,7 +263,7 @@ __device__ __forceinline__ void i8_tile(const I8Args& a, int e, int r0, int nr, 
                     float y = (static_cast<float>(i1) * rs) * ws1;
                     if (EPI == kI8Linear && a.bias) y = y + b1;
                     if (EPI == kI8Down) y = s_gate[m] * y;
-                    a.out[orow + col[1]] = y;
+                    a.out[orow + col1] = y;
                 }
             }
         }
@@ -281,12 +288,12 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(3))) void i
 // tile, column block) ordered column block by column block and cut into 8
 // contiguous parts the same way. Its blocks take the slots the routed units
 // leave free, so its own launch and the idle CUs of its small grid go.
-template <int EPI>
+template <int EPI, int NJ>
 __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(3))) void i8_grouped_kernel(
     I8Args a, const int* __restrict__ n_tiles, const int* __restrict__ tile_e, const int* __restrict__ tile_r0,
     const int* __restrict__ tile_nr, const int* __restrict__ exp_nt, const int* __restrict__ exp_t0, I8Args sh,
     int sh_rows, int sh_blocks) {
-    constexpr int BNB = bcols<EPI>();
+    constexpr int BNB = bcols<EPI, NJ>();
     int b = static_cast<int>(blockIdx.x);
     if (b < sh_blocks) {
         const int ncb_s = (sh.N + BNB - 1) / BNB;
@@ -297,7 +304,7 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(3))) void i
         const int gs = (b % kXcds) * per_s + ks;
         if (gs >= units_s) return;
         const int cb = gs / nt_s, r0 = (gs - cb * nt_s) * BM;
-        i8_tile<EPI>(sh, 0, r0, min(BM, sh_rows - r0), cb);
+        i8_tile<EPI, NJ>(sh, 0, r0, min(BM, sh_rows - r0), cb);
         return;
     }
     b -= sh_blocks;
@@ -312,7 +319,7 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(3))) void i
     const int loc = g - ncb * t0;
     const int cb = loc / nt;
     const int tile = t0 + (loc - cb * nt);
-    i8_tile<EPI>(a, e, tile_r0[tile], tile_nr[tile], cb);
+    i8_tile<EPI, NJ>(a, e, tile_r0[tile], tile_nr[tile], cb);
 }
 
 // One thread per 16-byte destination unit d = ((e * NT + nt) * KS + ks) * 64
@@ -376,17 +383,17 @@ hipError_t launch_moe_prefill_i8(hipStream_t s, const focr_hip_moe_layer* L, con
     }
     // sh_rows > 0: the dense product `sh` over that many rows rides in the
     // same launch (its blocks first, a multiple of 8 of them)
-    auto grouped = [&](auto epi, const I8Args& a, const I8Args& sh, int sh_rows) {
-        constexpr int EPI = decltype(epi)::value;
-        const int ncb = (a.N + bcols<EPI>() - 1) / bcols<EPI>();
+    auto grouped = [&](auto epi, auto nj, const I8Args& a, const I8Args& sh, int sh_rows) {
+        constexpr int EPI = decltype(epi)::value, NJ = decltype(nj)::value;
+        const int ncb = (a.N + bcols<EPI, NJ>() - 1) / bcols<EPI, NJ>();
         const int max_units = p.max_tiles * ncb;
         int sh_blocks = 0;
         if (sh_rows > 0) {
-            const int units_s = ((sh_rows + BM - 1) / BM) * ((sh.N + bcols<EPI>() - 1) / bcols<EPI>());
+            const int units_s = ((sh_rows + BM - 1) / BM) * ((sh.N + bcols<EPI, NJ>() - 1) / bcols<EPI, NJ>());
             sh_blocks = kXcds * ((units_s + kXcds - 1) / kXcds);
         }
         const dim3 grid(static_cast<unsigned>(sh_blocks + kXcds * ((max_units + kXcds - 1) / kXcds)));
-        FOCR_LAUNCH(i8_grouped_kernel<EPI>, grid, dim3(256), 0, s, a, p.n_tiles, p.tile_e, p.tile_r0, p.tile_nr,
+        FOCR_LAUNCH((i8_grouped_kernel<EPI, NJ>), grid, dim3(256), 0, s, a, p.n_tiles, p.tile_e, p.tile_r0, p.tile_nr,
                     p.exp_nt, p.exp_t0, sh, sh_rows, sh_blocks);
         return hipGetLastError();
     };
@@ -397,7 +404,7 @@ hipError_t launch_moe_prefill_i8(hipStream_t s, const focr_hip_moe_layer* L, con
         // the shared expert's gate/up (every token row, SwiGLU) as extra units
         const I8Args sh{w.xq, w.xs, nullptr, 1, L->swg_mfma, L->ssg, L->swu_mfma, L->ssu, nullptr, nullptr,
                         w.shared_act, H, SI};
-        if ((e = grouped(std::integral_constant<int, kI8Swiglu>(), a, sh, with_shared ? t : 0)) != hipSuccess)
+        if ((e = grouped(std::integral_constant<int, kI8Swiglu>(), std::integral_constant<int, 2>(), a, sh, with_shared ? t : 0)) != hipSuccess)
             return e;
     }
     {
@@ -419,11 +426,22 @@ hipError_t launch_moe_prefill_i8(hipStream_t s, const focr_hip_moe_layer* L, con
         // above), the prefill layer went 0.653 -> 0.629 ms at chunks of 256
         // and 0.310 -> 0.291 ms at one 1024-row chunk, although its units run
         // twice the K of the routed ones
+        // One column tile per wave (128-column blocks, twice as many, four
+        // stages of fragments in flight instead of two) while the 256-column
+        // blocks would not fill their three per CU: an expert's rows make
+        // about one 64-row tile plus one per 64 rows. Down launch with the
+        // shared expert, 256 -> 128 columns: 64 rows 28.8 -> 21.6 us, 256
+        // 29.3 -> 23.1, 512 30.6 -> 25.5, 768 37.4 -> 36.1, 1024 36.1 -> 36.8,
+        // 2048 57.4 -> 58.7.
+        const int est_tiles = std::min(E, TK) + TK / BM;
+        const bool narrow = est_tiles * ((H + 255) / 256) < 3 * ctx->cu_count;
         const I8Args a{w.aq, w.as, p.perm, top_k, L->wd_mfma, L->sd, nullptr, nullptr, nullptr, gates, w.ybuf, I, H};
         const I8Args sh{w.shared_aq, w.shared_as, nullptr, 1, L->swd_mfma, L->ssd, nullptr, nullptr, nullptr,
                         nullptr, w.shared_y, SI, H};
-        if ((e = grouped(std::integral_constant<int, kI8Down>(), a, sh, with_shared ? t : 0)) != hipSuccess)
-            return e;
+        const std::integral_constant<int, kI8Down> down;
+        e = narrow ? grouped(down, std::integral_constant<int, 1>(), a, sh, with_shared ? t : 0)
+                   : grouped(down, std::integral_constant<int, 2>(), a, sh, with_shared ? t : 0);
+        if (e != hipSuccess) return e;
     }
     {
         ProfScope ps(ctx, "i8_combine");

@@ -185,3 +185,37 @@ def test_moe_prefill_i8_bad_expert_index(ctx, gpu_layer):
     with pytest.raises(ContractViolation, match="expert index out of range"):
         gpu_layer.prefill(ctx.to_device(np.ones((t, H), np.float32)), ctx.to_device(idx),
                           ctx.to_device(np.ones((t, K), np.float32)), dout)
+
+
+@pytest.mark.parametrize("hidden,inter,si,t", [(192, 64, 320, 70), (320, 192, 64, 129), (1280, 896, 1792, 65)])
+def test_moe_prefill_i8_narrow_down_blocks(ctx, hidden, inter, si, t):
+    """Few rows take the down launch's 128-column blocks, the shared expert's
+    among them: hidden sizes that fill them partly (192, 320 = 2.5 blocks) and
+    K below, at and past a staged chunk, against the oracle (rel 1e-3, the MoE
+    output's tolerance)."""
+    from franken_ocr_amd.engine import MoeLayer
+
+    n_e, k = 5, 2
+    _say(f"moe prefill i8 narrow down H={hidden} I={inter} shared={si} t={t}")
+
+    def mat(seed, *shape):
+        return synth.int8_uniform(synth.seed_of(seed), int(np.prod(shape))).reshape(shape)
+
+    def sc(seed, *shape):
+        return synth.f32_uniform(synth.seed_of(seed), int(np.prod(shape)), 1e-3, 2e-2).reshape(shape)
+
+    router = synth.f32_normal(synth.seed_of(9700), n_e * hidden, 0.0, 0.02).reshape(n_e, hidden)
+    w = [mat(9701, n_e, inter, hidden), sc(9702, n_e, inter), mat(9703, n_e, inter, hidden), sc(9704, n_e, inter),
+         mat(9705, n_e, hidden, inter), sc(9706, n_e, hidden)]
+    sw = [mat(9707, si, hidden), sc(9708, si), mat(9709, si, hidden), sc(9710, si), mat(9711, hidden, si),
+          sc(9712, hidden)]
+    x = synth.f32_normal(synth.seed_of(9713), t * hidden).reshape(t, hidden)
+    idx, gates = synth.zipf_routing(synth.seed_of(9714), t, n_e, k)
+    layer = MoeLayer(hidden, inter, n_e, k, router, *w, ctx=ctx)
+    layer.set_shared(si, *sw)
+    out = ctx.empty((t, hidden), np.float32)
+    layer.prefill(ctx.to_device(x), ctx.to_device(idx), ctx.to_device(gates), out, with_shared=True)
+    flat = [a.reshape(-1) for a in w]
+    st, want = O.moe_prefill_i8(x, idx, gates, *flat, n_e, inter, shared=(si, *[a.reshape(-1) for a in sw]))
+    assert st == 0
+    assert_rel(out.numpy(), want, 1e-3)
