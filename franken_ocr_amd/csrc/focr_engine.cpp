@@ -1353,10 +1353,14 @@ int32_t rswa_write_all(focr_hip_ctx* ctx, focr_hip_rswa* c, const float* k_steps
     return FOCR_HIP_OK;
 }
 
-int32_t rswa_attend_all(focr_hip_ctx* ctx, const focr_hip_rswa* c, const float* q, float* out) {
+// step (= c) non-null: a whole step, the streams' new rows k_steps / v_steps
+// written to their rings by the attention's own launch and its cursors moved.
+int32_t rswa_attend_all(focr_hip_ctx* ctx, const focr_hip_rswa* c, const float* q, float* out,
+                        focr_hip_rswa* step = nullptr, const float* k_steps = nullptr,
+                        const float* v_steps = nullptr) {
     for (size_t s = 0; s < c->n_streams; ++s) {
         if (c->prefill_len[s] < 0) return fail(FOCR_HIP_E_STATE, "rswa: decode_attention before record_prefill");
-        if (c->prefill_len[s] + c->ring_len[s] == 0)
+        if (!step && c->prefill_len[s] + c->ring_len[s] == 0)
             return fail(FOCR_HIP_E_STATE, "rswa: empty attention key set (prefill_len=0, ring_len=0)");
     }
     if (!q || !out) return fail(FOCR_HIP_E_ARG, "rswa_decode_attention: null device pointer");
@@ -1370,10 +1374,16 @@ int32_t rswa_attend_all(focr_hip_ctx* ctx, const focr_hip_rswa* c, const float* 
         for (uint32_t i = 0; i < a.n; ++i) {
             a.prefill_len[i] = static_cast<uint32_t>(c->prefill_len[s0 + i]);
             a.ring_len[i] = c->ring_len[s0 + i];
+            if (step) {  // the keys after the write
+                a.slot[i] = peek_slot(c, s0 + i);
+                a.ring_len[i] = std::max(a.ring_len[i], a.slot[i] + 1);
+            }
         }
         const size_t off = s0 * kNumHeads * kHeadDim;
-        FOCR_HIP_TRY(launch_rswa_attention(ctx->stream, c, s0, a, q + off, out + off, partials, ctx->cu_count, ctx),
+        FOCR_HIP_TRY(launch_rswa_attention(ctx->stream, c, s0, a, q + off, out + off, partials, ctx,
+                                           step ? k_steps + off : nullptr, step ? v_steps + off : nullptr),
                      "attention launch");
+        for (uint32_t i = 0; step && i < a.n; ++i) advance_slot(step, s0 + i);
     }
     return FOCR_HIP_OK;
 }
@@ -1399,6 +1409,12 @@ int32_t focr_hip_rswa_step(focr_hip_ctx* ctx, focr_hip_rswa* c, const float* q, 
                            const float* v_steps, float* out) {
     ENGINE_CTX(ctx);
     if (!c) return fail(FOCR_HIP_E_BAD_HANDLE, "null rswa cache");
+    // the write inside the attention's launch, which reads the rows 16 bytes
+    // a lane; unaligned rows, and calls with something missing (as far as the
+    // two calls come), take the two calls
+    bool ready = q && out && k_steps && v_steps && aligned16(k_steps) && aligned16(v_steps);
+    for (size_t s = 0; s < c->n_streams; ++s) ready = ready && c->prefill_len[s] >= 0;
+    if (ready) return rswa_attend_all(ctx, c, q, out, c, k_steps, v_steps);
     int32_t st = rswa_write_all(ctx, c, k_steps, v_steps, nullptr);
     if (st) return st;
     return rswa_attend_all(ctx, c, q, out);

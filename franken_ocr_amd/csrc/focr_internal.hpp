@@ -653,6 +653,7 @@ hipError_t launch_rswa_write(hipStream_t s, const focr_hip_rswa* c, size_t s0,
 size_t rswa_partials_bytes(size_t n_streams, size_t max_keys);
 hipError_t launch_rswa_attention(hipStream_t s, const focr_hip_rswa* c, size_t s0,
                                  const RswaStepArgs& a, const float* q, float* out,
-                                 float* partials, int cu_count, focr_hip_ctx* ctx);
+                                 float* partials, focr_hip_ctx* ctx,
+                                 const float* k_steps = nullptr, const float* v_steps = nullptr);
 
 }  // namespace focr

@@ -216,3 +216,66 @@ def test_rswa_attention_across_cache_shapes(ctx):
                 assert np.array_equal(got, first[n]), shapes[n]
     for cache, *_ in setups:
         cache.free()
+
+
+def _ring_rows(ctx, cache, stream):
+    import ctypes as C
+
+    from franken_ocr_amd import _abi
+
+    reg = cache.regions(stream)
+    out = []
+    for key in ("ring_k", "ring_v"):
+        a = np.empty(NH * W * D, np.float32)
+        _abi.call("focr_hip_d2h", ctx.handle, a.ctypes.data_as(C.c_void_p), C.c_void_p(reg[key]), a.nbytes)
+        out.append(a)
+    return out
+
+
+@pytest.mark.parametrize("offset", [0, 4], ids=["aligned", "unaligned"])
+def test_rswa_step_equals_write_then_attention(ctx, offset):
+    """The step whose attention launch writes the rings gives the two calls'
+    outputs, rings and cursors bit for bit: prompts of 0 to 130 tokens (the
+    new key first, last and alone in its 64-key chunk), rings empty, partly
+    full, full and wrapped, and more streams than one launch takes; rows at an
+    unaligned address take the two launches."""
+    from franken_ocr_amd.engine import RingCache
+
+    cap = 130
+    states = [(p, n, r) for p in (0, 1, 63, 64, 130) for n, r in ((0, 0), (1, 1), (63, 63), (127, 127), (128, 0), (128, 127))]
+    states = (states * 3)[:70]
+    b = len(states)
+    _say(f"step against write + attention, {b} streams, offset {offset}")
+    rng = np.random.default_rng(77)
+    pair = [RingCache(b, cap, ctx) for _ in range(2)]
+    import ctypes as C
+
+    from franken_ocr_amd import _abi
+
+    for s, (p, n, r) in enumerate(states):
+        k, v = (ctx.to_device(rng.standard_normal((NH, max(p, 1), D), dtype=np.float32)) for _ in range(2))
+        rings = [rng.standard_normal(NH * W * D, dtype=np.float32) for _ in range(2)]
+        for cache in pair:
+            cache.record_prefill(s, k, v, p)
+            reg = cache.regions(s)
+            for key, a in zip(("ring_k", "ring_v"), rings):
+                _abi.call("focr_hip_h2d", ctx.handle, C.c_void_p(reg[key]), a.ctypes.data_as(C.c_void_p), a.nbytes)
+            cache.set_state(s, n, r)
+        ctx.synchronize()
+    outs = [ctx.empty((b, NH * D), np.float32) for _ in pair]
+    for step in range(2):
+        q = ctx.to_device(rng.standard_normal((b, NH * D), dtype=np.float32))
+        rows = []
+        for _ in range(2):
+            a = np.zeros(b * NH * D + 4, np.float32)
+            a[offset // 4:offset // 4 + b * NH * D] = rng.standard_normal(b * NH * D, dtype=np.float32)
+            rows.append(ctx.to_device(a))
+        ptrs = [r.offset(offset) for r in rows]
+        _abi.call("focr_hip_rswa_step", ctx.handle, pair[0]._h, q.c_ptr, ptrs[0], ptrs[1], outs[0].c_ptr)
+        _abi.call("focr_hip_rswa_write_decode_step", ctx.handle, pair[1]._h, ptrs[0], ptrs[1], None)
+        pair[1].decode_attention(q, outs[1])
+        assert np.array_equal(outs[0].numpy(), outs[1].numpy()), step
+        for s in range(b):
+            assert pair[0].state(s) == pair[1].state(s)
+            for x, y in zip(_ring_rows(ctx, pair[0], s), _ring_rows(ctx, pair[1], s)):
+                assert np.array_equal(x, y), (step, s)
