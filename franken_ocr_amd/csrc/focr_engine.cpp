@@ -829,14 +829,8 @@ int32_t moe_decode_impl(focr_hip_ctx* ctx, const focr_hip_moe_layer* L, const fl
             // products, scales and rounding as the expert's down projection
             // (decoder.rs:1753-1754), with the GEMV's full-grid weight stream
             ProfScope ps(ctx, "moe_shared_down");
-            const int SI = (int)L->shared_inter;
-            const int rows = 57344 / SI < 32 ? 57344 / SI : 32;  // the GEMV's activation stage: m * k <= 56 KiB
-            for (int r0 = 0; e == hipSuccess && r0 < (int)t; r0 += rows) {
-                const int mr = (int)t - r0 < rows ? (int)t - r0 : rows;
-                e = launch_gemv_i8_f32(str, L->swd, L->ssd, (int)L->hidden, SI, s.shared_act + (size_t)r0 * SI,
-                                       nullptr, 0.0f, mr, s.shared_y + (size_t)r0 * L->hidden,
-                                       s.shared_aq + (size_t)r0 * SI, s.shared_as + r0, ctx->cu_count);
-            }
+            e = launch_gemv_i8_f32(str, L->swd, L->ssd, (int)L->hidden, (int)L->shared_inter, s.shared_act, nullptr,
+                                   0.0f, (int)t, s.shared_y, s.shared_aq, s.shared_as, ctx->cu_count);
         }
     }
     if (e == hipSuccess && s.ybuf) {
@@ -1610,7 +1604,7 @@ static int32_t decoder_layer_step_impl(focr_hip_ctx* ctx, const focr_hip_decoder
         hipError_t qe = hipErrorNotSupported;
         if (L->qkv_rope_w) {
             ProfScope ps(ctx, "layer_qkv_rope");
-            const RopeEpi epi{L->inv_freq, rp, ring, q, (int)D, (int)L->head_dim, 0};
+            const RopeEpi epi{L->inv_freq, rp, ring, q, (int)D, (int)L->head_dim};
             qe = launch_qkv_rope_f32(s, L->qkv_rope_w, L->qkv_rope_s, (int)(3 * D), (int)H, x, L->input_ln, L->eps,
                                      (int)B, epi, ctx->cu_count);
             if (qe != hipErrorNotSupported) FOCR_HIP_TRY(qe, "qkv rope launch");
@@ -1652,7 +1646,7 @@ static int32_t decoder_layer_step_impl(focr_hip_ctx* ctx, const focr_hip_decoder
     // in one (h = x + attn stored by it); quantize_row_i8 of act; the down
     // GEMV with the residual add in its epilogue (x = h + down(act))
     const int cu = ctx->cu_count > 0 ? ctx->cu_count : 256;
-    if (!L->moe && L->gate_up_w && B >= 2 && H % 64 == 0 && H <= 1280 && I % 64 == 0 && I <= 8192 &&
+    if (!L->moe && L->gate_up_w && H % 64 == 0 && H <= 1280 && I % 64 == 0 && I <= 8192 &&
         (I + 15) / 16 < static_cast<size_t>(4 * cu) && (H + 15) / 16 < static_cast<size_t>(4 * cu)) {
         float* act = reinterpret_cast<float*>(take(B * I * 4));
         int8_t* aq = reinterpret_cast<int8_t*>(take(B * I));

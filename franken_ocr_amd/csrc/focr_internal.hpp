@@ -462,7 +462,7 @@ struct RopeRing {
 // The qkv GEMV's RoPE epilogue: the weights' q and k rows are in the pair
 // order of qkv_rope_row (each 16-row tile holds 8 (i, i + half) pairs of one
 // head), rows >= 2 D in order; q goes to q [rows][D], k and v to the ring
-// slots; row i of the launch is stream r0 + i.
+// slots; row i is stream i.
 struct RopeEpi {
     const float* inv_freq;
     RopePositions pos;
@@ -470,7 +470,6 @@ struct RopeEpi {
     float* q;
     int d_model;   // D = n_heads * head_dim
     int head_dim;
-    int r0;
 };
 // Original row of permuted qkv row p (p < 2 D: pairs; else p).
 __host__ __device__ inline int qkv_rope_row(int p, int D, int head_dim) {

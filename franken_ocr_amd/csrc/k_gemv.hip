@@ -303,7 +303,8 @@ struct IgemmMode {
     int accumulate;
     size_t sw, sx, so;
     // row groups (the split-K kernel, rows > 0): blockIdx.y takes activation
-    // rows [16 y, 16 y + 16) of `rows`; y and a_scales advance by sy / sa
+    // rows [16 y, 16 y + 16) of `rows`; y and a_scales advance by sy / sa,
+    // f32 rows and residual rows by 16 of their own
     size_t sy, sa;
     int rows;
 };
@@ -558,17 +559,28 @@ __global__ __launch_bounds__(kThreads) void gemv_i8_mfma_splitk_kernel(
     const int8_t* __restrict__ W, const float* __restrict__ ws, int N, int K, const int8_t* __restrict__ xq,
     const float* __restrict__ a_scales, int M, float* __restrict__ y, int32_t* __restrict__ acc_out,
     const float* __restrict__ xf, const float* __restrict__ nw, float eps, RopeEpi re, const IgemmMode im,
-    const RowAdd radd) {
+    RowAdd radd) {
     static_assert(!ADD || (FQ && !ROPE), "ADD is an f32-input form");
     static_assert(!SWIGLU || !ROPE, "one epilogue");
     extern __shared__ int4 lds_dyn[];  // x [M][K/16 + 1], then per-wave [16][16] chunks
+    [[maybe_unused]] int rope_r0 = 0;  // the row group's first stream
     if (gridDim.y > 1) {
         W += blockIdx.y * im.sw;
         xq += blockIdx.y * im.sx;
         acc_out += blockIdx.y * im.so;
         if (y) y += blockIdx.y * im.sy;
         if (a_scales) a_scales += blockIdx.y * im.sa;
-        if (im.rows > 0) M = min(16, im.rows - 16 * static_cast<int>(blockIdx.y));  // block-uniform
+        if (im.rows > 0) {  // block-uniform
+            const int r0 = 16 * static_cast<int>(blockIdx.y);
+            M = min(16, im.rows - r0);
+            if constexpr (FQ) xf += static_cast<size_t>(r0) * K;
+            if constexpr (ADD) {
+                radd.xf2 += static_cast<size_t>(r0) * K;
+                radd.h_out += static_cast<size_t>(r0) * K;
+            }
+            rope_r0 = r0;
+            if (radd.resid) radd.resid += static_cast<size_t>(r0) * N;
+        }
     }
     __shared__ v4i_m red[kThreads / 64][64];
     __shared__ v4i_m red_u[SWIGLU ? kThreads / 64 : 1][64];  // SWIGLU: the up tile's partials
@@ -782,7 +794,7 @@ __global__ __launch_bounds__(kThreads) void gemv_i8_mfma_splitk_kernel(
             const float yv = (static_cast<float>(acc[v]) * lds_as[i]) * wscale;
             const float pv = __int_as_float(dpp_mov<0xB1>(__float_as_int(yv)));  // lane col ^ 1: the pair partner
             if (i >= M || n >= N) continue;
-            const int s = re.r0 + i;
+            const int s = rope_r0 + i;
             if (n < 2 * D) {
                 const int part = n / D, pl = n - part * D;
                 const int hd = pl / hdim, pr = pl - hd * hdim;
@@ -951,39 +963,59 @@ hipError_t launch_quantize_rows2(hipStream_t s, const QuantRows& r1, const Quant
     return hipGetLastError();
 }
 
+// The split-K kernel's forms over m rows in groups of 16 on grid.y: one
+// launch where one per group ran them one after another (the MoE layer with
+// the shared expert at 29 rows 86.6 -> 77.2 us, at 64 rows 122.8 -> 96.7; a
+// decode step of 17 streams 1685 -> 1460 us). One row takes them too: the
+// sdot4 kernel is as fast on the weights, but needs a quantize (and norm)
+// launch of its own before it, and the RoPE and dense-MLP forms exist only
+// here (a decode step of one stream 664 -> 584 us).
+static IgemmMode row_groups(int m, int n) {
+    IgemmMode im{};
+    im.sy = static_cast<size_t>(16) * n;
+    im.sa = 16;
+    im.rows = m;
+    return im;
+}
+static size_t splitk_lds(int m, int k) {
+    return (static_cast<size_t>(m < 16 ? m : 16) * (k / 16 + 1) + (kThreads / 64) * kMfmaTileBytes / 16) * sizeof(int4);
+}
+// The n columns (of 16 per block) leave CUs idle, the staged rows fit LDS.
+static bool splitk_fits(int m, int n, int k, int cu_count) {
+    const size_t lds_static = (kThreads / 64) * 64 * sizeof(int4) * 2 + 16 * sizeof(float);
+    return m >= 1 && m <= 16 * 65535 && k >= 64 && k % 64 == 0 && splitk_lds(m, k) + lds_static <= max_lds_per_block() &&
+           (n + 15) / 16 < 4 * (cu_count > 0 ? cu_count : 256);
+}
+static bool aligned_f4(const void* p) { return reinterpret_cast<uintptr_t>(p) % 16 == 0; }
+
 hipError_t launch_gemv_i8_f32(hipStream_t s, const int8_t* w, const float* ws, int n, int k, const float* x,
                               const float* norm_w, float eps, int m, float* y, int8_t* xq_tmp, float* xs_tmp,
                               int cu_count) {
     if (m < 1 || k <= 0) return hipErrorInvalidValue;
-    const size_t lds_splitk =
-        (static_cast<size_t>(m < 16 ? m : 16) * (k / 16 + 1) + (kThreads / 64) * kMfmaTileBytes / 16) * sizeof(int4);
-    const size_t lds_splitk_static = (kThreads / 64) * 64 * sizeof(int4) + 16 * sizeof(float);
-    if (m >= kMfmaMinRows && k % 64 == 0 && k <= kFqMaxK && lds_splitk + lds_splitk_static <= max_lds_per_block() &&
-        (n + 15) / 16 < 4 * (cu_count > 0 ? cu_count : 256)) {
-        const int grid = (n + 15) / 16;
-        for (int r0 = 0; r0 < m; r0 += 16) {
-            const int mr = m - r0 < 16 ? m - r0 : 16;
-            if (k <= 64 * 4 * 5)  // rows of <= 5 float4 per lane
-                FOCR_LAUNCH((gemv_i8_mfma_splitk_kernel<2, true, false, 5>), dim3(grid), dim3(kThreads), lds_splitk,
-                            s, w, ws, n, k, nullptr, nullptr, mr, y + static_cast<size_t>(r0) * n, nullptr,
-                            x + static_cast<size_t>(r0) * k, norm_w, eps, RopeEpi{}, IgemmMode{}, RowAdd{});
-            else if (k <= 64 * 4 * 7)  // <= 7 (the shared expert's 1792-wide act rows)
-                FOCR_LAUNCH((gemv_i8_mfma_splitk_kernel<2, true, false, 7>), dim3(grid), dim3(kThreads), lds_splitk,
-                            s, w, ws, n, k, nullptr, nullptr, mr, y + static_cast<size_t>(r0) * n, nullptr,
-                            x + static_cast<size_t>(r0) * k, norm_w, eps, RopeEpi{}, IgemmMode{}, RowAdd{});
-            else
-                FOCR_LAUNCH((gemv_i8_mfma_splitk_kernel<2, true>), dim3(grid), dim3(kThreads), lds_splitk, s, w, ws,
-                            n, k, nullptr, nullptr, mr, y + static_cast<size_t>(r0) * n, nullptr,
-                            x + static_cast<size_t>(r0) * k, norm_w, eps, RopeEpi{}, IgemmMode{}, RowAdd{});
-        }
+    if (k <= kFqMaxK && splitk_fits(m, n, k, cu_count) && aligned_f4(x) && aligned_f4(norm_w)) {
+        const dim3 grid((n + 15) / 16, (m + 15) / 16);
+        const size_t lds = splitk_lds(m, k);
+        const IgemmMode im = row_groups(m, n);
+        const int mr = m < 16 ? m : 16;
+        if (k <= 64 * 4 * 5)  // rows of <= 5 float4 per lane
+            FOCR_LAUNCH((gemv_i8_mfma_splitk_kernel<2, true, false, 5>), grid, dim3(kThreads), lds, s, w, ws, n, k,
+                        nullptr, nullptr, mr, y, nullptr, x, norm_w, eps, RopeEpi{}, im, RowAdd{});
+        else if (k <= 64 * 4 * 7)  // <= 7 (the shared expert's 1792-wide act rows)
+            FOCR_LAUNCH((gemv_i8_mfma_splitk_kernel<2, true, false, 7>), grid, dim3(kThreads), lds, s, w, ws, n, k,
+                        nullptr, nullptr, mr, y, nullptr, x, norm_w, eps, RopeEpi{}, im, RowAdd{});
+        else
+            FOCR_LAUNCH((gemv_i8_mfma_splitk_kernel<2, true>), grid, dim3(kThreads), lds, s, w, ws, n, k, nullptr,
+                        nullptr, mr, y, nullptr, x, norm_w, eps, RopeEpi{}, im, RowAdd{});
         return hipGetLastError();
     }
     // otherwise: the norm / quantize kernel, then the GEMV on the int8 rows
+    // (its activation stage holds 56 KiB)
     hipError_t e = norm_w ? launch_rms_norm_quant(s, x, norm_w, m, k, eps, xq_tmp, xs_tmp)
                           : launch_quantize_rows(s, x, m, k, xq_tmp, xs_tmp, 0);
     if (e != hipSuccess) return e;
-    for (int r0 = 0; r0 < m && e == hipSuccess; r0 += 32) {
-        const int mr = m - r0 < 32 ? m - r0 : 32;
+    const int rows = 57344 / k < 1 ? 1 : 57344 / k < 32 ? 57344 / k : 32;
+    for (int r0 = 0; r0 < m && e == hipSuccess; r0 += rows) {
+        const int mr = m - r0 < rows ? m - r0 : rows;
         e = launch_gemv_i8(s, w, ws, n, k, xq_tmp + static_cast<size_t>(r0) * k, xs_tmp + r0, mr,
                            y + static_cast<size_t>(r0) * n, nullptr, nullptr, nullptr, cu_count);
     }
@@ -994,49 +1026,32 @@ hipError_t launch_swiglu_i8_f32_add(hipStream_t s, const int8_t* w_gu, const flo
                                     const float* x, const float* x2, float* h_out, const float* norm_w, float eps,
                                     int m, float* act, int cu_count) {
     if (m < 1 || !x2 || !h_out) return hipErrorInvalidValue;
-    const size_t lds_splitk =
-        (static_cast<size_t>(m < 16 ? m : 16) * (k / 16 + 1) + (kThreads / 64) * kMfmaTileBytes / 16) * sizeof(int4);
-    const size_t lds_splitk_static = (kThreads / 64) * 64 * sizeof(int4) + 16 * sizeof(float);
-    if (m < kMfmaMinRows || k < 64 || k % 64 != 0 || k > 64 * 4 * 5 ||
-        lds_splitk + lds_splitk_static > max_lds_per_block() || (n + 15) / 16 >= 4 * (cu_count > 0 ? cu_count : 256))
-        return hipErrorNotSupported;
-    const int grid = (n + 15) / 16;
-    for (int r0 = 0; r0 < m; r0 += 16) {
-        const int mr = m - r0 < 16 ? m - r0 : 16;
-        const size_t off = static_cast<size_t>(r0) * k;
-        FOCR_LAUNCH((gemv_i8_mfma_splitk_kernel<2, true, false, 5, true, true>), dim3(grid), dim3(kThreads),
-                    lds_splitk, s, w_gu, ws_gu, n, k, nullptr, nullptr, mr, act + static_cast<size_t>(r0) * n, nullptr,
-                    x + off, norm_w, eps, RopeEpi{}, IgemmMode{}, RowAdd{x2 + off, h_out + off, nullptr});
-    }
+    if (k > 64 * 4 * 5 || !splitk_fits(m, n, k, cu_count) || !aligned_f4(x)) return hipErrorNotSupported;
+    FOCR_LAUNCH((gemv_i8_mfma_splitk_kernel<2, true, false, 5, true, true>), dim3((n + 15) / 16, (m + 15) / 16),
+                dim3(kThreads), splitk_lds(m, k), s, w_gu, ws_gu, n, k, nullptr, nullptr, m < 16 ? m : 16, act, nullptr,
+                x, norm_w, eps, RopeEpi{}, row_groups(m, n), RowAdd{x2, h_out, nullptr});
     return hipGetLastError();
 }
 
 hipError_t launch_gemv_i8_resid(hipStream_t s, const int8_t* w, const float* ws, int n, int k, const int8_t* xq,
                                 const float* a_scales, int m, const float* resid, float* y, int cu_count) {
     if (m < 1 || !resid) return hipErrorInvalidValue;
-    const size_t lds_splitk =
-        (static_cast<size_t>(m < 16 ? m : 16) * (k / 16 + 1) + (kThreads / 64) * kMfmaTileBytes / 16) * sizeof(int4);
-    const size_t lds_splitk_static = (kThreads / 64) * 64 * sizeof(int4) + 16 * sizeof(float);
-    if (m < kMfmaMinRows || k < 64 || k % 64 != 0 || k > 256 * 4 * kSplitKMaxChunks ||
-        lds_splitk + lds_splitk_static > max_lds_per_block() || (n + 15) / 16 >= 4 * (cu_count > 0 ? cu_count : 256))
-        return hipErrorNotSupported;
-    const int grid = (n + 15) / 16;
-    const int cpw = ((k + 255) / 256 + 3) / 4;
-    for (int r0 = 0; r0 < m; r0 += 16) {
-        const int mr = m - r0 < 16 ? m - r0 : 16;
-        const int8_t* xq_r = xq + static_cast<size_t>(r0) * k;
-        float* y_r = y + static_cast<size_t>(r0) * n;
-        const RowAdd ra{nullptr, nullptr, resid + static_cast<size_t>(r0) * n};
-        if (cpw <= 2)
-            FOCR_LAUNCH((gemv_i8_mfma_splitk_kernel<2, false>), dim3(grid), dim3(kThreads), lds_splitk, s, w, ws, n,
-                        k, xq_r, a_scales + r0, mr, y_r, nullptr, nullptr, nullptr, 0.0f, RopeEpi{}, IgemmMode{}, ra);
-        else if (cpw <= 4)
-            FOCR_LAUNCH((gemv_i8_mfma_splitk_kernel<4, false>), dim3(grid), dim3(kThreads), lds_splitk, s, w, ws, n,
-                        k, xq_r, a_scales + r0, mr, y_r, nullptr, nullptr, nullptr, 0.0f, RopeEpi{}, IgemmMode{}, ra);
-        else
-            FOCR_LAUNCH((gemv_i8_mfma_splitk_kernel<8, false>), dim3(grid), dim3(kThreads), lds_splitk, s, w, ws, n,
-                        k, xq_r, a_scales + r0, mr, y_r, nullptr, nullptr, nullptr, 0.0f, RopeEpi{}, IgemmMode{}, ra);
-    }
+    if (k > 256 * 4 * kSplitKMaxChunks || !splitk_fits(m, n, k, cu_count)) return hipErrorNotSupported;
+    const dim3 grid((n + 15) / 16, (m + 15) / 16);
+    const size_t lds = splitk_lds(m, k);
+    const int cpw = ((k + 255) / 256 + 3) / 4, mr = m < 16 ? m : 16;
+    IgemmMode im = row_groups(m, n);
+    im.sx = static_cast<size_t>(16) * k;
+    const RowAdd ra{nullptr, nullptr, resid};
+    if (cpw <= 2)
+        FOCR_LAUNCH((gemv_i8_mfma_splitk_kernel<2, false>), grid, dim3(kThreads), lds, s, w, ws, n, k, xq, a_scales, mr,
+                    y, nullptr, nullptr, nullptr, 0.0f, RopeEpi{}, im, ra);
+    else if (cpw <= 4)
+        FOCR_LAUNCH((gemv_i8_mfma_splitk_kernel<4, false>), grid, dim3(kThreads), lds, s, w, ws, n, k, xq, a_scales, mr,
+                    y, nullptr, nullptr, nullptr, 0.0f, RopeEpi{}, im, ra);
+    else
+        FOCR_LAUNCH((gemv_i8_mfma_splitk_kernel<8, false>), grid, dim3(kThreads), lds, s, w, ws, n, k, xq, a_scales, mr,
+                    y, nullptr, nullptr, nullptr, 0.0f, RopeEpi{}, im, ra);
     return hipGetLastError();
 }
 
@@ -1103,30 +1118,22 @@ hipError_t launch_permute_rows_i8(hipStream_t s, const int8_t* w, const float* w
 
 hipError_t launch_qkv_rope_f32(hipStream_t s, const int8_t* w_perm, const float* ws_perm, int n, int k,
                                const float* x, const float* norm_w, float eps, int m, RopeEpi epi, int cu_count) {
-    const size_t lds_splitk =
-        (static_cast<size_t>(m < 16 ? m : 16) * (k / 16 + 1) + (kThreads / 64) * kMfmaTileBytes / 16) * sizeof(int4);
-    const size_t lds_splitk_static = (kThreads / 64) * 64 * sizeof(int4) + 16 * sizeof(float);
     const int D = epi.d_model;
-    if (m < kMfmaMinRows || m > RopePositions::kMax || k < 64 || k % 64 != 0 || k > kFqMaxK || n != 3 * D ||
-        epi.head_dim % 16 != 0 || D % epi.head_dim != 0 || !epi.q || !epi.inv_freq ||
-        lds_splitk + lds_splitk_static > max_lds_per_block() || (n + 15) / 16 >= 4 * (cu_count > 0 ? cu_count : 256))
+    if (m > RopePositions::kMax || k > kFqMaxK || n != 3 * D || epi.head_dim % 16 != 0 || D % epi.head_dim != 0 ||
+        !epi.q || !epi.inv_freq || !splitk_fits(m, n, k, cu_count) || !aligned_f4(x) || !aligned_f4(norm_w))
         return hipErrorNotSupported;
     for (int i = 0; i < m; ++i)
         if (!epi.ring.k[i] || !epi.ring.v[i]) return hipErrorInvalidValue;
-    const int grid = (n + 15) / 16;
-    for (int r0 = 0; r0 < m; r0 += 16) {
-        const int mr = m - r0 < 16 ? m - r0 : 16;
-        RopeEpi e = epi;
-        e.r0 = r0;
-        if (k <= 64 * 4 * 5)  // rows of <= 5 float4 per lane
-            FOCR_LAUNCH((gemv_i8_mfma_splitk_kernel<2, true, true, 5>), dim3(grid), dim3(kThreads), lds_splitk, s,
-                        w_perm, ws_perm, n, k, nullptr, nullptr, mr, nullptr, nullptr,
-                        x + static_cast<size_t>(r0) * k, norm_w, eps, e, IgemmMode{}, RowAdd{});
-        else
-            FOCR_LAUNCH((gemv_i8_mfma_splitk_kernel<2, true, true>), dim3(grid), dim3(kThreads), lds_splitk, s,
-                        w_perm, ws_perm, n, k, nullptr, nullptr, mr, nullptr, nullptr,
-                        x + static_cast<size_t>(r0) * k, norm_w, eps, e, IgemmMode{}, RowAdd{});
-    }
+    const dim3 grid((n + 15) / 16, (m + 15) / 16);
+    const size_t lds = splitk_lds(m, k);
+    const IgemmMode im = row_groups(m, n);
+    const int mr = m < 16 ? m : 16;
+    if (k <= 64 * 4 * 5)  // rows of <= 5 float4 per lane
+        FOCR_LAUNCH((gemv_i8_mfma_splitk_kernel<2, true, true, 5>), grid, dim3(kThreads), lds, s, w_perm, ws_perm, n, k,
+                    nullptr, nullptr, mr, nullptr, nullptr, x, norm_w, eps, epi, im, RowAdd{});
+    else
+        FOCR_LAUNCH((gemv_i8_mfma_splitk_kernel<2, true, true>), grid, dim3(kThreads), lds, s, w_perm, ws_perm, n, k,
+                    nullptr, nullptr, mr, nullptr, nullptr, x, norm_w, eps, epi, im, RowAdd{});
     return hipGetLastError();
 }
 

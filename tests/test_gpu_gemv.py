@@ -125,3 +125,29 @@ def test_argmax_rows_edge_cases(ctx):
     argmax_rows(d, da)
     want = [O.argmax_row(r)[1] for r in rows]
     assert da.numpy().tolist() == want == [100, 0, 77777, want[3], 0, n - 1]
+
+
+@pytest.mark.parametrize("m", [1, 15, 16, 17, 32])
+@pytest.mark.parametrize("offset", [0, 4], ids=["aligned", "unaligned"])
+def test_gemv_i8_row_groups(ctx, m, offset):
+    """One launch over the row groups of 16 (one row, a full group, one row
+    past it, two groups), and rows at an address that 16-byte loads cannot
+    take: bit-exact against the oracle, with a NaN row among them."""
+    import ctypes as C
+
+    from franken_ocr_amd import _abi
+    from franken_ocr_amd.engine import QInt8
+
+    n, k = 1288, 1280  # 80.5 column blocks
+    _say(f"gemv rows m={m} offset={offset}")
+    w, s = _weights(n, k, 30)
+    x = synth.f32_normal(synth.seed_of(31 + m), m * k).reshape(m, k)
+    x[m // 2, 5] = np.nan
+    host = np.zeros(m * k + 4, np.float32)
+    host[offset // 4:offset // 4 + m * k] = x.reshape(-1)
+    dx = ctx.to_device(host)
+    q = QInt8(w, s, n, k, ctx)
+    dy = ctx.empty((m, n), np.float32)
+    _abi.call("focr_hip_gemv_i8", ctx.handle, q.handle, C.c_void_p(dx.ptr + offset), m, dy.c_ptr)
+    want = O.gemv_i8_batched(x, w, s, n, k)[0]
+    assert np.array_equal(dy.numpy(), want)
