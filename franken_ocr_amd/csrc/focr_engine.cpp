@@ -823,7 +823,10 @@ int32_t moe_decode_impl(focr_hip_ctx* ctx, const focr_hip_moe_layer* L, const fl
         // call's route would take this call's records for its own
         if (e != hipSuccess) launch_route_epoch_bump(str, s.xchg);
     }
-    if (e == hipSuccess && with_shared) {
+    // few rows: the shared expert's down product rides in the down + combine
+    const bool shared_in_down = with_shared && !s.ybuf &&
+                                moe_down_combine_takes_shared(d, (int)L->inter, (int)L->shared_inter);
+    if (e == hipSuccess && with_shared && !shared_in_down) {
         {
             // quantize_row_i8 of the act rows, then the int8 GEMV: the same
             // products, scales and rounding as the expert's down projection
@@ -844,8 +847,9 @@ int32_t moe_decode_impl(focr_hip_ctx* ctx, const focr_hip_moe_layer* L, const fl
         }
     } else if (e == hipSuccess) {
         ProfScope ps(ctx, "moe_down_combine");
+        const MoeSharedDown shd{s.shared_act, L->swd, L->ssd};
         e = launch_moe_down_combine(str, d, di, dg, s.flag, s.act, L->wd, L->sd, with_shared ? s.shared_y : nullptr,
-                                    resid, out, (int)L->inter);
+                                    resid, out, (int)L->inter, shared_in_down ? &shd : nullptr);
     }
     if (e != hipSuccess) return hip_fail(e, "moe_decode launch");
     if (check_route) return check_route_flags(ctx, s.flag, t, token_base);

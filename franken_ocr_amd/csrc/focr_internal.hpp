@@ -406,9 +406,18 @@ constexpr int kMoeMaxT = 64;
 constexpr int kLayerPrefillMaxRows = 4096;  // rows of one decoder_layer_prefill chunk
 // down + slot-order combine in one launch, reading the routing from idx /
 // gates / flag ([t][top_k]) and the act rows of every pair (t*top_k + j).
+// The shared expert's down product for the down + combine launch: its act
+// rows [t][2 * inter] (f32), weights [hidden][2 * inter] and row scales.
+struct MoeSharedDown {
+    const float* act;
+    const int8_t* wd;
+    const float* sd;
+};
+bool moe_down_combine_takes_shared(const MoeDims& d, int inter, int shared_inter);
 hipError_t launch_moe_down_combine(hipStream_t s, const MoeDims& d, const uint32_t* idx, const float* gates,
                                    const int* flag, const float* act, const int8_t* wd, const float* sd,
-                                   const float* shared_y, const float* resid, float* out, int inter);
+                                   const float* shared_y, const float* resid, float* out, int inter,
+                                   const MoeSharedDown* shared = nullptr);
 // k_attn.hip — causal prefill attention on the f32 matrix cores (head_dim
 // 128). Element (row i, head h) of q / out and (key j, head h) of k / v sit at
 // base + i * ld + h * hstride (token-major: ld = heads * 128, hstride = 128).

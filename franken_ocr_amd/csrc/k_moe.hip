@@ -892,16 +892,28 @@ __global__ __launch_bounds__(256) void moe_down_kernel(
 // A weight row used by several of the step's tokens is read once per token;
 // such blocks run together (t varies fastest), so the repeats mostly hit the
 // caches.
+//
+// SH (few tokens, a shared expert of twice the routed width, RPG 1): the
+// shared expert's down product in the same blocks, its launch gone. A wave
+// without a slot quantizes its act row; each of the block's R rows is two
+// half-row dots for lane groups 0 .. 2R - 1, whose i32 sums add up to the
+// whole row's (exactly). The 28 more weight registers leave two blocks per CU
+// (128 blocks a token), so it pays while every block is resident: the layer
+// with the shared expert at 1 / 2 / 3 / 4 tokens 21.2 / 24.4 / 28.0 / 30.3 ->
+// 18.4 / 21.5 / 25.7 / 28.2 us, at 5 and 6 tokens 34.1 / 35.9 -> 33.5 / 35.7,
+// where a launch of its own stays; a decode step of one stream 593 -> 551 us.
 constexpr int DC_THREADS = 512;
 
-template <int LPR, int JC, int RPG>
-__global__ __launch_bounds__(DC_THREADS) void moe_down_combine_kernel(
+template <int LPR, int JC, int RPG, bool SH = false>
+__global__ __launch_bounds__(DC_THREADS) __attribute__((amdgpu_waves_per_eu(SH ? 4 : 2))) void moe_down_combine_kernel(
     const uint32_t* __restrict__ idx, const float* __restrict__ gates, const int* __restrict__ flag, int T, int K,
     const float* __restrict__ act, const int8_t* __restrict__ wd, const float* __restrict__ sd,
     const float* __restrict__ shared_y, const float* __restrict__ resid, float* __restrict__ out, int H, int I,
-    int E) {
-    extern __shared__ int4 lds_q[];  // [K][I/16] quantized act rows of token t
-    __shared__ float s_as[kMaxK];
+    int E, MoeSharedDown shd) {
+    static_assert(!SH || RPG == 1, "the shared rows take the second row's registers");
+    extern __shared__ int4 lds_q[];  // [K][I/16] quantized act rows of token t (SH: then the shared row)
+    __shared__ float s_as[kMaxK + 1];
+    __shared__ int s_sh[SH ? DC_THREADS / LPR : 1];
     constexpr int NG = DC_THREADS / LPR;
     __shared__ float s_y[RPG * NG];
     // XCD-aware order: blocks are dispatched to the 8 XCDs round-robin
@@ -938,14 +950,24 @@ __global__ __launch_bounds__(DC_THREADS) void moe_down_combine_kernel(
     }
     const int bad = flag[t];
     const bool qwave = wave < K;  // wave-uniform
-    const float* ar = act + static_cast<size_t>(t * K + (qwave ? wave : 0)) * I;
-    const bool short_row = I <= 64 * NQ;
-    float v[NQ];
+    const bool swave = SH && wave == K;  // the shared act row's wave (2 I values)
+    const float* ar = swave ? shd.act + static_cast<size_t>(t) * 2 * I
+                            : act + static_cast<size_t>(t * K + (qwave ? wave : 0)) * I;
+    const int len = swave ? 2 * I : I;
+    const bool short_row = SH || I <= 64 * NQ;
+    float v[NQ], v2[SH ? NQ : 1];  // v2: the shared row's values past 64 NQ
     if (short_row) {
 #pragma unroll
         for (int q = 0; q < NQ; ++q) {
             const int i = wl + 64 * q;
-            v[q] = ar[i < I ? i : I - 1];  // a duplicate of the last value past I: max unchanged
+            v[q] = ar[i < len ? i : len - 1];  // a duplicate of the last value past I: max unchanged
+        }
+        if constexpr (SH) {
+#pragma unroll
+            for (int q = 0; q < NQ; ++q) {
+                const int i = wl + 64 * (NQ + q);
+                v2[q] = ar[i < len ? i : len - 1];
+            }
         }
     }
     // 2. the down rows of the group's pairs
@@ -960,19 +982,36 @@ __global__ __launch_bounds__(DC_THREADS) void moe_down_combine_kernel(
         for (int c = 0; c < JC; ++c) wv[q][c] = row_chunk(drow, ln + LPR * c, C);
         sdr[q] = sd[row];
     }
+    // SH: group g's half row of the shared down matrix (row rb * R + g / 2)
+    int4 ws[SH ? JC : 1];
+    if constexpr (SH) {
+        const int r = g < 2 * R && rb * R + g / 2 < H ? rb * R + g / 2 : 0;
+        const int4* drow = reinterpret_cast<const int4*>(shd.wd + static_cast<size_t>(r) * 2 * I + (g & 1) * I);
+#pragma unroll
+        for (int c = 0; c < JC; ++c) ws[c] = row_chunk(drow, ln + LPR * c, C);
+    }
     // 3. quantize_row_i8 of the act rows into LDS
-    if (qwave) {
+    if (qwave || swave) {
         int8_t* qrow = reinterpret_cast<int8_t*>(lds_q) + wave * I;
         if (short_row) {
             float amax = 0.0f;
 #pragma unroll
             for (int q = 0; q < NQ; ++q) amax = fmaxf(amax, fabsf(v[q]));
+            if constexpr (SH) {
+#pragma unroll
+                for (int q = 0; q < NQ; ++q) amax = fmaxf(amax, fabsf(v2[q]));
+            }
             amax = wave_max_f_full(amax);
             const float a_scale = amax > 0.0f ? amax / 127.0f : 1.0f;
             const float inv = 1.0f / a_scale;
 #pragma unroll
             for (int q = 0; q < NQ; ++q)
-                if (wl + 64 * q < I) qrow[wl + 64 * q] = quant_i8(v[q], inv, false);
+                if (wl + 64 * q < len) qrow[wl + 64 * q] = quant_i8(v[q], inv, false);
+            if constexpr (SH) {
+#pragma unroll
+                for (int q = 0; q < NQ; ++q)
+                    if (wl + 64 * (NQ + q) < len) qrow[wl + 64 * (NQ + q)] = quant_i8(v2[q], inv, false);
+            }
             if (wl == 0) s_as[wave] = a_scale;
         } else {  // long rows: two passes over L2
             float amax = 0.0f;
@@ -996,6 +1035,16 @@ __global__ __launch_bounds__(DC_THREADS) void moe_down_combine_kernel(
         d = reduce_lanes<LPR>(d);
         if (ln == 0) s_y[g + NG * q] = ((static_cast<float>(d) * s_as[jq[q]]) * sdr[q]) * gate[q];
     }
+    if constexpr (SH) {
+        int d = 0;
+#pragma unroll
+        for (int c = 0; c < JC; ++c) {
+            const int cc = ln + LPR * c;
+            if (cc < C) d = dot16_i8(ws[c], lds_q[(K + (g & 1)) * C + cc], d);
+        }
+        d = reduce_lanes<LPR>(d);
+        if (ln == 0) s_sh[g] = d;
+    }
     __syncthreads();
     // 4. slot-order sum of the token's K results for each row
     if (threadIdx.x < R) {
@@ -1004,7 +1053,10 @@ __global__ __launch_bounds__(DC_THREADS) void moe_down_combine_kernel(
             float o = 0.0f;
             if (!bad) {
                 for (int jj = 0; jj < K; ++jj) o += s_y[threadIdx.x * K + jj];
-                if (shared_y) o += shared_y[static_cast<size_t>(t) * H + rr];
+                if constexpr (SH)
+                    o += (static_cast<float>(s_sh[2 * threadIdx.x] + s_sh[2 * threadIdx.x + 1]) * s_as[K]) * shd.sd[rr];
+                else if (shared_y)
+                    o += shared_y[static_cast<size_t>(t) * H + rr];
             }
             if (resid) o = resid[static_cast<size_t>(t) * H + rr] + o;  // h + mlp_out (decoder.rs:2625)
             out[static_cast<size_t>(t) * H + rr] = o;
@@ -1227,9 +1279,21 @@ hipError_t launch_moe_combine(hipStream_t s, const MoeDims& d, const float* ybuf
     return hipGetLastError();
 }
 
+constexpr int kSharedDownTokens = 4;
+
+bool moe_down_combine_takes_shared(const MoeDims& d, int inter, int shared_inter) {
+    int lpr, jc;
+    pick_lpr(inter, &lpr, &jc);
+    // a free wave for the shared act row, a free lane group pair per row, the
+    // row in NQ registers a lane, and every block resident (two per CU)
+    return d.t <= kSharedDownTokens && shared_inter == 2 * inter && lpr == 8 && jc == 7 && inter <= 64 * NQ &&
+           d.top_k < DC_THREADS / 64 && 2 * (DC_THREADS / lpr / d.top_k) <= DC_THREADS / lpr;
+}
+
 hipError_t launch_moe_down_combine(hipStream_t s, const MoeDims& d, const uint32_t* idx, const float* gates,
                                    const int* flag, const float* act, const int8_t* wd, const float* sd,
-                                   const float* shared_y, const float* resid, float* out, int inter) {
+                                   const float* shared_y, const float* resid, float* out, int inter,
+                                   const MoeSharedDown* shared) {
     int lpr, jc;
     pick_lpr(inter, &lpr, &jc);
     if (!dims_ok(d) || inter % 16 != 0 || jc > 8) return hipErrorInvalidValue;
@@ -1246,11 +1310,17 @@ hipError_t launch_moe_down_combine(hipStream_t s, const MoeDims& d, const uint32
     const int rpg = two_ok && d.t * row_blocks(1) > 768 ? 2 : 1;
     const int nrb8 = row_blocks(rpg);
     const dim3 grid(static_cast<unsigned>(d.t * nrb8));
-    const size_t lds = static_cast<size_t>(d.top_k) * inter;
+    const size_t lds = static_cast<size_t>(d.top_k + (shared ? 2 : 0)) * inter;
+    if (shared) {
+        const dim3 sgrid(static_cast<unsigned>(d.t * row_blocks(1)));
+        FOCR_LAUNCH((moe_down_combine_kernel<8, 7, 1, true>), sgrid, dim3(DC_THREADS), lds, s, idx, gates, flag, d.t,
+                    d.top_k, act, wd, sd, nullptr, resid, out, d.hidden, inter, d.n_experts, *shared);
+        return hipGetLastError();
+    }
 #define FOCR_DC(L, J, P)                                                                                          \
     if (lpr == L && jc == J && rpg == P) {                                                                       \
         FOCR_LAUNCH((moe_down_combine_kernel<L, J, P>), grid, dim3(DC_THREADS), lds, s, idx, gates, flag, d.t,   \
-                    d.top_k, act, wd, sd, shared_y, resid, out, d.hidden, inter, d.n_experts);                   \
+                    d.top_k, act, wd, sd, shared_y, resid, out, d.hidden, inter, d.n_experts, MoeSharedDown{});  \
         return hipGetLastError();                                                                                \
     }
     FOCR_DC(8, 1, 1) FOCR_DC(8, 2, 1) FOCR_DC(8, 3, 1) FOCR_DC(8, 4, 1) FOCR_DC(8, 5, 1) FOCR_DC(8, 6, 1)

@@ -353,3 +353,41 @@ def test_route_fallback_when_the_other_blocks_are_not_waited_for(layer_w, t):
     assert st == 0 and np.array_equal(res[1][0], want_i)
     layer.free()
     c.close()
+
+
+@pytest.mark.parametrize("h,inter,e,k", [(1280, 896, 64, 6), (208, 800, 6, 2), (336, 896, 9, 7)])
+def test_moe_shared_down_inside_down_combine(ctx, h, inter, e, k):
+    """Up to four tokens with a shared expert of twice the routed width take
+    the shared down product inside the down + combine launch: each token's row
+    is the same, bit for bit, as in a call of eight tokens (a launch of its
+    own), with a token that has no finite score among them, and matches the
+    oracle (rel 1e-3). Rows that do not fill the last row block, one lane
+    group pair per row or fewer, and a half row of 50 chunks."""
+    from franken_ocr_amd.engine import MoeLayer
+
+    si = 2 * inter
+    router = synth.f32_normal(synth.seed_of(700), e * h, 0.0, 0.05).reshape(e, h)
+    w = [a for n, kk, sd in ((inter, h, 701), (inter, h, 703), (h, inter, 705))
+         for a in (synth.int8_uniform(synth.seed_of(sd), e * n * kk),
+                   synth.f32_uniform(synth.seed_of(sd + 1), e * n, 1e-3, 2e-2))]
+    sw = [a for n, kk, sd in ((si, h, 711), (si, h, 713), (h, si, 715))
+          for a in (synth.int8_uniform(synth.seed_of(sd), n * kk),
+                    synth.f32_uniform(synth.seed_of(sd + 1), n, 1e-3, 2e-2))]
+    layer = MoeLayer(h, inter, e, k, router, *w, ctx=ctx)
+    layer.set_shared(si, *sw)
+    x = synth.f32_normal(synth.seed_of(720), 8 * h).reshape(8, h)
+    x[2, 3] = np.nan
+
+    def run(rows):
+        out = ctx.empty(rows.shape, np.float32)
+        layer.decode(ctx.to_device(rows), out, with_shared=True, check_route=False)
+        return out.numpy()
+
+    whole = run(x)
+    for t in range(1, 6):
+        _say(f"shared down inside down + combine: {t} tokens of {h} x {inter}, {e} experts, top {k}")
+        assert np.array_equal(run(x[:t]), whole[:t]), t
+    good = np.array([0, 1, 3, 4])
+    st, want, _, _ = O.moe_decode(x[good], router, *w, e, k, inter, shared=(si, *sw))
+    assert st == 0
+    assert_rel(whole[good], want, 1e-3)
