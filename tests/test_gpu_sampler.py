@@ -199,3 +199,30 @@ def test_sampler_errors(ctx):
     # NaN temperature is greedy (sampler.rs:96-100)
     sample_rows(rows, tok, ngram_size=0, temperature=math.nan)
     assert tok.numpy().tolist() == [0, 0]
+
+
+@pytest.mark.parametrize("n", [2, 8, 9, 10, 17, 18])
+def test_long_windows_and_compare_groups(ctx, n):
+    """Windows on both sides of the 4096 tokens held on chip, and n-grams whose
+    n - 1 tokens end before, on and after a group of eight: whole numbers, so
+    the pick is the oracle's exactly."""
+    rng = np.random.default_rng(n)
+    rows, seqs = [], []
+    for L in (n - 1, n, n + 1, 4095, 4096, 4097, 6000):
+        pre = rng.integers(8, 100, n - 1).tolist()
+        body = rng.integers(8, 100, max(L - n, 0)).tolist()
+        near = list(pre)
+        near[-1] += 100  # differs in its last token alone: bans nothing
+        seq = (pre + [7] + body)[: max(L - (n - 1), 0)] + pre
+        if L > 4 * n:
+            seq[2 * n : 3 * n] = near + [6]
+        row = np.zeros(256, np.float32)
+        row[6], row[7] = 9.0, 10.0
+        rows.append(row)
+        seqs.append(seq)
+    for window in (0, 4096, 5000):
+        _say(f"n={n} window={window}")
+        tok, _ = _sample_dev(ctx, rows, seqs, n, window)
+        for i, seq in enumerate(seqs):
+            st, want, _ = O.sample(rows[i], np.asarray(seq, np.uint32), n, window)
+            assert st == 0 and tok[i] == want, (n, window, len(seq))
