@@ -602,13 +602,14 @@ size_t attn_partials_bytes(int cs, int heads, int nsplit) {
 int attn_pick_splits(int cs, int c1, int heads, int cu_count, int* split_len) {
     // Row tile i (kRT rows) needs the tiles of keys [0, min(c1, c0 + kRT (i + 1))):
     // ranges of `per` tiles give sum over i of ceil(n_i / per) blocks per
-    // head. The length taken is the one with the least estimated time, from
-    // per-block timestamps (us): a block alone on its CU spends 5.8 on its
-    // query rows, first tile and output and 3.1 a tile; two on a CU 10 and
-    // 3.7; more run in rounds. The partials of the ranges are written and
-    // read back at about 5 TB/s, and the merge is a launch of its own. At
-    // 1024 rows 3 tiles (510 blocks) took 35 us where 2 and 6 took 42 and 40;
-    // for 256 rows after 768 keys 3 (220 blocks) 23.5, 2 (320) 27.5, 4 26.9.
+    // head. The length taken is the one with the least estimated time (us),
+    // fitted to whole calls of 16 to 1280 rows at 1 to 16 tiles a range: 3.0 a
+    // tile where each block has a CU alone, 2 + 4.2 a tile where two share
+    // one, more in rounds of that; with more than one range, the partials
+    // written and read back at 6.6 TB/s and 11.5 for the merge launch and its
+    // tail. Measured calls at the length taken and its neighbours: 1024 rows 3
+    // tiles 36.2, 2 43.5, 4 38.2, 7 38.1; 768 rows 4 28.2, 3 32.8, 5 30.7; 256
+    // rows after 768 keys 3 23.5, 2 27.5, 4 26.9; 2048 rows 12 83.7, 8 96.5.
     const int c0 = c1 - cs;
     const double cus = cu_count > 0 ? cu_count : 1;
     const int tiles = (c1 + kKT - 1) / kKT;
@@ -621,8 +622,8 @@ int attn_pick_splits(int cs, int c1, int heads, int cu_count, int* split_len) {
             blocks += static_cast<double>(ranges) * heads;
             part_rows += static_cast<double>(ranges) * heads * min(kRT, cs - r);
         }
-        double us = blocks <= cus ? 5.8 + 3.1 * p : ceil(blocks / (kBlocksPerCu * cus)) * (10.0 + 3.7 * p);
-        if (p < tiles) us += 4.0 + part_rows * (kD + 2) * sizeof(float) * 2 / 5e6;
+        double us = blocks <= cus ? 3.0 * p : ceil(blocks / (kBlocksPerCu * cus)) * (2.0 + 4.2 * p);
+        if (p < tiles) us += 11.5 + part_rows * (kD + 2) * sizeof(float) * 2 / 6.6e6;
         if (best == 0.0 || us < best) {
             best = us;
             per = p;
