@@ -472,16 +472,16 @@ __global__ void route_epoch_bump_kernel(RouteXchg* __restrict__ xch) {
 // token's XCD L2), which is what a 256-1024-row chunk pays for. Here a block
 // holds two router rows per wave in registers (eight experts) and runs them
 // against kRowsTB token rows staged in LDS (all their loads in flight at
-// once): the router is read once per kRowsTB tokens (4 up to 512 rows, where
-// the blocks are few, else 8). Each logit is route_dots' f64 dot in the same
+// once): the router is read once per kRowsTB tokens. Each logit is route_dots' f64 dot in the same
 // lane order (lane l: float4 chunks l + 64 i, x, y, z, w in turn) and the
 // same DPP tree, so the logits are the split route's bit for bit;
 // route_rank_kernel then runs the split route's own softmax / top-k
 // (route_rank) on them, one wave per token. The f64 FMAs, converts and DPP
-// trees bound it (about 10 us of VALU at 1024 rows). Rows up to 1280
-// wide (one batch of kRouteNC float4 per lane); no exchange buffer, no
-// quantized rows.
-template <int kRowsTB>
+// trees bound it (about 10 us of VALU at 1024 rows, where the matrix-core
+// kernel below takes over). Rows up to 1280 wide (one batch of kRouteNC float4
+// per lane); no exchange buffer, no quantized rows.
+constexpr int kRowsTB = 4;
+
 __global__ __launch_bounds__(256) void route_logits_kernel(const float* __restrict__ x, const float* __restrict__ G,
                                                            int T, int H, int E, float* __restrict__ logits) {
     // the block's kRowsTB token rows, staged at once (every load in flight
@@ -549,6 +549,65 @@ __global__ __launch_bounds__(256) void route_logits_kernel(const float* __restri
             logits[static_cast<size_t>(t) * E + e0 + lane] = static_cast<float>(lane == 0 ? d[0] : d[1]);
     }
 }
+
+// The same logits for more rows: a block is 16 tokens x 16 experts on
+// v_mfma_f64_16x16x4, so each f32 operand is converted once per 16 partners
+// and the reduction trees go; one round of loads and the matrix pipe bound it.
+// K is split over the block's 8 waves, 32 floats (a cache line of each row) at
+// a time; the waves' f64 partials meet in LDS and are rounded to f32 once, as
+// above (the f64 sums run in another order). Lane l holds row (token or
+// expert) l % 16 and, of each 16-float group, the four at 4 (l / 16): MFMA j
+// of the group takes element j of both, a permutation of K that the two
+// operands share. C element v of lane l is token 4 v + l / 16, expert l % 16.
+// Few rows leave it few blocks; the kernel above and this one (us, 64 experts,
+// 1280 floats): 256 rows 6.1, 6.9; 320 7.4, 7.3; 384 8.5, 7.2; 512 10.0, 7.4;
+// 1024 15.3 (13.2 with 8 tokens a block), 7.5 to 8.8; 4096 47.6, 23.6.
+typedef double v4d __attribute__((ext_vector_type(4)));
+constexpr int kLogitWaves = 8;
+constexpr int kLogitMfmaT = 320;  // rows from which it is taken
+
+__global__ __launch_bounds__(64 * kLogitWaves) void route_logits_mfma_kernel(const float* __restrict__ x,
+                                                                            const float* __restrict__ G, int T, int H,
+                                                                            int E, float* __restrict__ logits) {
+    __shared__ double s_part[kLogitWaves][4][64];
+    const int wave = threadIdx.x >> 6;
+    const int lane = threadIdx.x & 63;
+    const int r = lane & 15, q = lane >> 4;
+    const int H4 = H >> 2;
+    const int t0 = 16 * static_cast<int>(blockIdx.x), e0 = 16 * static_cast<int>(blockIdx.y);
+    // rows past the end repeat the last one, never stored
+    const float4* xr = reinterpret_cast<const float4*>(x + static_cast<size_t>(min(t0 + r, T - 1)) * H);
+    const float4* gr = reinterpret_cast<const float4*>(G + static_cast<size_t>(min(e0 + r, E - 1)) * H);
+    float4 xv[2 * kRouteNC], gv[2 * kRouteNC];
+    unsigned m[2 * kRouteNC];
+#pragma unroll
+    for (int i = 0; i < 2 * kRouteNC; ++i) {
+        const int c = 4 * (2 * (wave + kLogitWaves * (i >> 1)) + (i & 1)) + q;
+        m[i] = c < H4 ? 0xFFFFFFFFu : 0u;
+        xv[i] = xr[c < H4 ? c : H4 - 1];
+        gv[i] = gr[c < H4 ? c : H4 - 1];
+    }
+    auto keep = [](float v, unsigned mask) { return static_cast<double>(__uint_as_float(__float_as_uint(v) & mask)); };
+    v4d acc = {0.0, 0.0, 0.0, 0.0};
+#pragma unroll
+    for (int i = 0; i < 2 * kRouteNC; ++i) {
+        acc = __builtin_amdgcn_mfma_f64_16x16x4f64(keep(xv[i].x, m[i]), keep(gv[i].x, m[i]), acc, 0, 0, 0);
+        acc = __builtin_amdgcn_mfma_f64_16x16x4f64(keep(xv[i].y, m[i]), keep(gv[i].y, m[i]), acc, 0, 0, 0);
+        acc = __builtin_amdgcn_mfma_f64_16x16x4f64(keep(xv[i].z, m[i]), keep(gv[i].z, m[i]), acc, 0, 0, 0);
+        acc = __builtin_amdgcn_mfma_f64_16x16x4f64(keep(xv[i].w, m[i]), keep(gv[i].w, m[i]), acc, 0, 0, 0);
+    }
+#pragma unroll
+    for (int v = 0; v < 4; ++v) s_part[wave][v][lane] = acc[v];
+    __syncthreads();
+    if (threadIdx.x < 256) {
+        const int v = wave, t = t0 + 4 * v + q, e = e0 + r;
+        double d = s_part[0][v][lane];
+#pragma unroll
+        for (int w = 1; w < kLogitWaves; ++w) d += s_part[w][v][lane];
+        if (t < T && e < E) logits[static_cast<size_t>(t) * E + e] = static_cast<float>(d);
+    }
+}
+static_assert(32 * kLogitWaves * kRouteNC == 64 * 4 * kRouteNC, "the waves cover the widest row");
 
 // One wave per token: its E logits (lane = expert) through route_rank.
 __global__ __launch_bounds__(256) void route_rank_kernel(const float* __restrict__ logits, int T, int E, int K,
@@ -1213,13 +1272,15 @@ hipError_t launch_moe_route_rows(hipStream_t s, const MoeDims& d, const float* h
     if (d.t < 1 || d.t > kRouteMaxT || d.n_experts < 1 || d.n_experts > kMaxE || d.top_k < 1 ||
         d.top_k > kMaxK || d.top_k > d.n_experts || !moe_route_rows_supported(d.hidden) || !logits)
         return hipErrorInvalidValue;
-    const unsigned parts = static_cast<unsigned>((d.n_experts + kRouteEPP - 1) / kRouteEPP);
-    if (d.t <= 512)
-        FOCR_LAUNCH(route_logits_kernel<4>, dim3(static_cast<unsigned>((d.t + 3) / 4), parts), dim3(256), 0, s,
-                    hidden, router, d.t, d.hidden, d.n_experts, logits);
+    if (d.t < kLogitMfmaT)
+        FOCR_LAUNCH(route_logits_kernel,
+                    dim3(static_cast<unsigned>((d.t + kRowsTB - 1) / kRowsTB),
+                         static_cast<unsigned>((d.n_experts + kRouteEPP - 1) / kRouteEPP)),
+                    dim3(256), 0, s, hidden, router, d.t, d.hidden, d.n_experts, logits);
     else
-        FOCR_LAUNCH(route_logits_kernel<8>, dim3(static_cast<unsigned>((d.t + 7) / 8), parts), dim3(256), 0, s,
-                    hidden, router, d.t, d.hidden, d.n_experts, logits);
+        FOCR_LAUNCH(route_logits_mfma_kernel,
+                    dim3(static_cast<unsigned>((d.t + 15) / 16), static_cast<unsigned>((d.n_experts + 15) / 16)),
+                    dim3(64 * kLogitWaves), 0, s, hidden, router, d.t, d.hidden, d.n_experts, logits);
     hipError_t e = hipGetLastError();
     if (e != hipSuccess) return e;
     FOCR_LAUNCH(route_rank_kernel, dim3(static_cast<unsigned>((d.t + 3) / 4)), dim3(256), 0, s, logits, d.t,

@@ -391,3 +391,30 @@ def test_moe_shared_down_inside_down_combine(ctx, h, inter, e, k):
     st, want, _, _ = O.moe_decode(x[good], router, *w, e, k, inter, shared=(si, *sw))
     assert st == 0
     assert_rel(whole[good], want, 1e-3)
+
+
+@pytest.mark.parametrize("t,e,k,h", [(319, 64, 6, 1280), (320, 64, 6, 1280), (321, 64, 6, 1280), (400, 33, 4, 1264), (513, 16, 3, 272),
+                                     (401, 1, 1, 16)])
+def test_route_matrix_core_logits(ctx, t, e, k, h):
+    """The f64 matrix-core logits at ends of the 16 x 16 tiles and of the waves'
+    K shares (1264 and 272 floats: a last line that is partly past the row; 16:
+    one wave with half a line). Both sides sum in f64 and round once, so a logit
+    differs by at most one f32 rounding; a probability then by that times the
+    largest logit magnitude (below 8 here), relatively: 8 x 2 x 2^-24 < 1e-6."""
+    from franken_ocr_amd.engine import MoeLayer
+
+    _say(f"route t={t} e={e} h={h}")
+    router = synth.f32_normal(synth.seed_of(950 + h), e * h, 0.0, 0.02).reshape(e, h)
+    x = synth.f32_normal(synth.seed_of(951 + t), t * h).reshape(t, h)
+    inter = 64
+    wg, wu = (synth.int8_uniform(synth.seed_of(952 + i), e * inter * h).reshape(e, inter, h) for i in range(2))
+    wd = synth.int8_uniform(synth.seed_of(954), e * h * inter).reshape(e, h, inter)
+    L = MoeLayer(h, inter, e, k, router, wg, np.ones((e, inter), np.float32), wu, np.ones((e, inter), np.float32),
+                 wd, np.ones((e, h), np.float32), ctx=ctx)
+    didx, dg, dp = ctx.empty((t, k), np.uint32), ctx.empty((t, k), np.float32), ctx.empty((t, e), np.float32)
+    L.route(ctx.to_device(x), didx, dg, dp, norm_topk=True)
+    st, idx, w, probs = O.route(x, router, e, k, norm_topk=True)
+    assert st == 0
+    assert np.array_equal(didx.numpy(), np.asarray(idx).reshape(t, k))
+    np.testing.assert_allclose(dp.numpy(), np.asarray(probs).reshape(t, e), rtol=1e-6, atol=1e-12)
+    np.testing.assert_allclose(dg.numpy(), np.asarray(w).reshape(t, k), rtol=2e-6, atol=0)
