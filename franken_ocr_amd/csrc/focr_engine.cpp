@@ -1072,22 +1072,36 @@ int32_t ensure_tiled(focr_hip_ctx* ctx, int8_t** dst, const int8_t* src, size_t 
 
 extern "C" {
 
+// Which kernel an int8 product of m rows takes: the tiled-order GEMMs from 256
+// rows on; below, without a bias, the split-K GEMV in 16-row groups on the
+// upload layout where it is the faster, else 64-row tiles on the fragment-order
+// weight copy. At 256 rows, the GEMV's last size, it took 10.8 us for 1280 x
+// 1280 where the tiled order's 64 x 64 blocks take 6.8; it stays there for a
+// call captured into a graph before the handle has its tiled weights, which
+// cannot be allocated then.
+static bool linear_i8_rows_gemv(focr_hip_ctx* ctx, const focr_hip_qint8* w, size_t m, const float* bias) {
+    if (bias || !gemv_rows_preferred((int)w->n, (int)w->k, (int)m, false)) return false;
+    if (!i8_gemm256_supported((int)m, (int)w->n, (int)w->k)) return true;
+    if (w->w_tiled) return false;
+    hipStreamCaptureStatus cap = hipStreamCaptureStatusNone;
+    return hipStreamIsCapturing(ctx->stream, &cap) != hipSuccess || cap != hipStreamCaptureStatusNone;
+}
+
 // norm_w (nullable): x is first RMS-normalised with that weight and eps, in
-// the quantize launch; only on the 256 x 128 tiled path (the caller checks
+// the quantize launch; only on the tiled path (the caller checks
 // linear_i8_norm_fusable)
-static bool linear_i8_norm_fusable(const focr_hip_qint8* w, size_t m) {
-    return w && !gemv_rows_preferred((int)w->n, (int)w->k, (int)m, false) &&
-           i8_gemm256_supported((int)m, (int)w->n, (int)w->k) && w->k <= 4096;
+static bool linear_i8_norm_fusable(focr_hip_ctx* ctx, const focr_hip_qint8* w, size_t m) {
+    return w && !linear_i8_rows_gemv(ctx, w, m, nullptr) && i8_gemm256_supported((int)m, (int)w->n, (int)w->k) &&
+           w->k <= 4096;
 }
 
 // The activation layout linear_int8_dynamic quantizes x into (row-major, or
-// the 256 x 128 GEMM's tiled order) and its bytes, in the kScrXq slot.
-static bool linear_i8_act_tiled(const focr_hip_qint8* w, size_t m, const float* bias) {
-    if (!bias && gemv_rows_preferred((int)w->n, (int)w->k, (int)m, false)) return false;
-    return i8_gemm256_supported((int)m, (int)w->n, (int)w->k);
+// the tiled order) and its bytes, in the kScrXq slot.
+static bool linear_i8_act_tiled(focr_hip_ctx* ctx, const focr_hip_qint8* w, size_t m, const float* bias) {
+    return !linear_i8_rows_gemv(ctx, w, m, bias) && i8_gemm256_supported((int)m, (int)w->n, (int)w->k);
 }
-static size_t linear_i8_act_bytes(const focr_hip_qint8* w, size_t m, const float* bias) {
-    return linear_i8_act_tiled(w, m, bias) ? i8_gemm256_a_bytes((int)m, (int)w->k) : m * w->k;
+static size_t linear_i8_act_bytes(focr_hip_ctx* ctx, const focr_hip_qint8* w, size_t m, const float* bias) {
+    return linear_i8_act_tiled(ctx, w, m, bias) ? i8_gemm256_a_bytes((int)m, (int)w->k) : m * w->k;
 }
 
 // prequant: the rows are already quantized by the dynamic rule in the
@@ -1101,12 +1115,9 @@ static int32_t linear_i8_dynamic_impl(focr_hip_ctx* ctx, const focr_hip_qint8* w
     if (!i8_mfma_supported(static_cast<int>(w->k)))
         return fail(FOCR_HIP_E_SHAPE,
                     fmt("linear_int8_dynamic: k %zu is not a multiple of 64 (the matrix-core K stage)", w->k));
-    // up to 256 rows without a bias, where it is the faster: the split-K GEMV
-    // in 16-row groups on the upload layout (a prefill chunk's o_proj gets 10
-    // blocks of the tiled GEMM at this size, (n / 16) x (m / 16) here)
-    if (norm_w && !linear_i8_norm_fusable(w, m))
+    if (norm_w && !linear_i8_norm_fusable(ctx, w, m))
         return fail(FOCR_HIP_E_ARG, "linear_int8_dynamic: the fused norm needs the tiled path");
-    if (!bias && gemv_rows_preferred((int)w->n, (int)w->k, (int)m, false)) {
+    if (linear_i8_rows_gemv(ctx, w, m, bias)) {
         int8_t* xq = static_cast<int8_t*>(ctx->scratch_get(kScrXq, m * w->k));
         float* xs = static_cast<float*>(ctx->scratch_get(kScrXs, m * sizeof(float)));
         if (!xq || !xs) return FOCR_HIP_E_OOM;
@@ -1120,8 +1131,6 @@ static int32_t linear_i8_dynamic_impl(focr_hip_ctx* ctx, const focr_hip_qint8* w
                      "linear_i8 launch");
         return FOCR_HIP_OK;
     }
-    // 256 rows and up: 256 x 128 LDS-staged tiles on the tiled operands;
-    // fewer: 64-row tiles on the fragment-order weight copy
     const bool big = i8_gemm256_supported((int)m, (int)w->n, (int)w->k);
     if (big) {
         if (!w->w_tiled) {
@@ -1160,7 +1169,7 @@ static int32_t linear_i8_dynamic_impl(focr_hip_ctx* ctx, const focr_hip_qint8* w
     ProfScope ps(ctx, "linear_i8");
     if (big)
         FOCR_HIP_TRY(launch_i8_gemm256(ctx->stream, xq, xs, (int)m, (int)w->k, w->w_tiled, w->scales, (int)w->n,
-                                       bias, y),
+                                       bias, y, ctx->cu_count),
                      "linear_i8 launch");
     else
         FOCR_HIP_TRY(launch_linear_i8(ctx->stream, xq, xs, (int)m, (int)w->k, w->w_mfma, w->scales, (int)w->n, bias,
@@ -1866,7 +1875,7 @@ static int32_t decoder_layer_prefill_impl(focr_hip_ctx* ctx, const focr_hip_deco
     //    reference block and the chunk's causal attention over [0, c0 + cs)
     // the input norm inside qkv's quantize launch where qkv takes the tiled GEMM
     // (its float4 row loads need 16-byte aligned rows and norm weight)
-    if (linear_i8_norm_fusable(L->qkv, cs) && reinterpret_cast<uintptr_t>(x) % 16 == 0 &&
+    if (linear_i8_norm_fusable(ctx, L->qkv, cs) && reinterpret_cast<uintptr_t>(x) % 16 == 0 &&
         reinterpret_cast<uintptr_t>(L->input_ln) % 16 == 0 && H % 4 == 0) {
         if ((st = linear_i8_dynamic_impl(ctx, L->qkv, x, cs, nullptr, qkv, L->input_ln, L->eps))) return st;
     } else {
@@ -1888,8 +1897,8 @@ static int32_t decoder_layer_prefill_impl(focr_hip_ctx* ctx, const focr_hip_deco
     // the split merge writes the context rows quantized for o_proj, in the
     // layout and scratch o_proj's linear_int8_dynamic reads
     AttnQuantOut qo{};
-    qo.tiled = linear_i8_act_tiled(L->o_proj, cs, nullptr);
-    qo.xq = static_cast<int8_t*>(ctx->scratch_get(kScrXq, linear_i8_act_bytes(L->o_proj, cs, nullptr)));
+    qo.tiled = linear_i8_act_tiled(ctx, L->o_proj, cs, nullptr);
+    qo.xq = static_cast<int8_t*>(ctx->scratch_get(kScrXq, linear_i8_act_bytes(ctx, L->o_proj, cs, nullptr)));
     qo.xs = static_cast<float*>(ctx->scratch_get(kScrXs, cs * sizeof(float)));
     if (!qo.xq || !qo.xs) return FOCR_HIP_E_OOM;
     if ((st = rswa_prefill_chunk_impl(ctx, cache, stream, q, nullptr, nullptr, cs, c0, cx, true, &qo))) return st;

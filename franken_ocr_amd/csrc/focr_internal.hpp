@@ -594,7 +594,7 @@ hipError_t launch_quantize_rows_tiled(hipStream_t s, const float* x, int m, int 
 hipError_t launch_rms_norm_quantize_rows_tiled(hipStream_t s, const float* x, const float* nw, float eps, int m,
                                               int k, int8_t* xt, float* xs, int rule);
 hipError_t launch_i8_gemm256(hipStream_t s, const int8_t* xt, const float* xs, int m, int k, const int8_t* wt,
-                             const float* ws, int n, const float* bias, float* y);
+                             const float* ws, int n, const float* bias, float* y, int cu_count);
 struct MoeI8Scratch {
     int8_t* xq;       // [t][hidden]
     float* xs;        // [t]

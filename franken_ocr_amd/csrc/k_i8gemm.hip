@@ -259,6 +259,127 @@ __global__ __launch_bounds__(NTHR) __attribute__((amdgpu_waves_per_eu(WPE, WPE))
     }
 }
 
+// The same product where 256 x 128 blocks would leave CUs idle (a prefill
+// chunk's attention projections): 64 x 64 blocks, whose four waves split K by
+// stages (wave w takes stages w, w + 4, ..) and meet in LDS; the i32 sums are
+// exact in any order, so the values are the large blocks'. Both operands come
+// straight from the tiled order into registers (a wave's fragment load is 16
+// bytes of each of 32 rows, 64 bytes apart: the stage's two K steps use up the
+// lines between them), kSmRing stages in flight a wave: at K = 1280 that is
+// everything a block reads, in one round of latency, and no barrier until the
+// sums meet (256 rows of 3840 x 1280: 15.6 us in the large blocks, 7.7 here;
+// bound by that latency). Blocks are ordered column block by column block and
+// cut into 8 contiguous parts, one per XCD, so each weight slab is read by one
+// L2.
+constexpr int SM = 64, SN = 64;  // block rows / columns
+constexpr int kSmRing = 5;       // stages in flight per wave
+constexpr int kSmXcds = 8;
+
+__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2, 2))) void i8_gemm64_kernel(const GemmArgs a) {
+    __shared__ v4i s_part[4][3][4][64];  // [tile][other wave][4 elements][lane]
+    __shared__ float s_rs[SM], s_ws[SN], s_b[SN];
+    const int nrt = (a.M + SM - 1) / SM, units = nrt * ((a.N + SN - 1) / SN);
+    const int per = (units + kSmXcds - 1) / kSmXcds;
+    const int g = static_cast<int>(blockIdx.x) % kSmXcds * per + static_cast<int>(blockIdx.x) / kSmXcds;
+    if (g >= units) return;  // block-uniform
+    const int m0 = g % nrt * SM, n0 = g / nrt * SN;
+    const int tid = threadIdx.x;
+    const int wave = __builtin_amdgcn_readfirstlane(tid >> 6), l = tid & 63;
+    const int h = l >> 5, c32 = l & 31;
+    const int nst = a.K / BK;
+    const bool has_bias = a.bias != nullptr;
+    if (tid < SM) {
+        s_rs[tid] = a.a_scale[min(m0 + tid, a.M - 1)];
+    } else if (tid < SM + SN) {
+        const int col = min(n0 + tid - SM, a.N - 1);
+        s_ws[tid - SM] = a.w_scale[col];
+        s_b[tid - SM] = has_bias ? a.bias[col] : 0.0f;
+    }
+
+    // stage st of the block's 64 rows: 4 KB inside the row tile's stage
+    const int8_t* ga = a.A + static_cast<size_t>(m0 / TM) * nst * TM * BK + m0 % TM * BK;
+    const int8_t* gb = a.B + static_cast<size_t>(n0 / TN) * nst * TN * BK + n0 % TN * BK;
+    int off[2];  // K step s: piece 2 s + h of row c32 (swz has the same value 32 rows on)
+#pragma unroll
+    for (int s = 0; s < 2; ++s) off[s] = c32 * BK + 16 * ((2 * s + h) ^ swz(c32));
+    struct Frag {
+        v4i a[2][2], b[2][2];  // [row / column tile][K step]
+    };
+    auto load = [&](int i, Frag& f) {
+        const int st = min(wave + 4 * i, nst - 1);
+        const int8_t* pa = ga + static_cast<size_t>(st) * TM * BK;
+        const int8_t* pb = gb + static_cast<size_t>(st) * TN * BK;
+#pragma unroll
+        for (int t = 0; t < 2; ++t)
+#pragma unroll
+            for (int s = 0; s < 2; ++s) {
+                f.a[t][s] = *reinterpret_cast<const v4i*>(pa + 32 * BK * t + off[s]);
+                f.b[t][s] = *reinterpret_cast<const v4i*>(pb + 32 * BK * t + off[s]);
+            }
+    };
+    v16i acc[2][2] = {};
+    // a stage past K (i >= the wave's count) adds zeros
+    auto compute = [&](int i, const Frag& f) {
+        const bool live = wave + 4 * i < nst;
+        const v4i z = {0, 0, 0, 0};
+#pragma unroll
+        for (int s = 0; s < 2; ++s)
+#pragma unroll
+            for (int u = 0; u < 2; ++u) {
+                const v4i b = live ? f.b[u][s] : z;
+#pragma unroll
+                for (int t = 0; t < 2; ++t)
+                    acc[t][u] = __builtin_amdgcn_mfma_i32_32x32x32_i8(f.a[t][s], b, acc[t][u], 0, 0, 0);
+            }
+    };
+    Frag f[kSmRing];
+#pragma unroll
+    for (int q = 0; q < kSmRing; ++q) load(q, f[q]);
+    const int count = (nst + 3) / 4;  // stages of wave 0, the most of any
+    int i = 0;
+    for (; i + kSmRing < count; i += kSmRing) {
+#pragma unroll
+        for (int q = 0; q < kSmRing; ++q) {
+            compute(i + q, f[q]);
+            __builtin_amdgcn_sched_barrier(0);  // the refill after its products
+            load(i + kSmRing + q, f[q]);
+            __builtin_amdgcn_sched_barrier(0);
+        }
+    }
+#pragma unroll
+    for (int q = 0; q < kSmRing; ++q) compute(i + q, f[q]);
+
+    // wave w finishes tile (w / 2, w % 2): the others hand it their sums
+    auto part = [&](const v16i& v, int q) { return v4i{v[4 * q], v[4 * q + 1], v[4 * q + 2], v[4 * q + 3]}; };
+    v4i sum[4];
+#pragma unroll
+    for (int t = 0; t < 4; ++t)
+#pragma unroll
+        for (int q = 0; q < 4; ++q) {
+            if (t == wave)
+                sum[q] = part(acc[t >> 1][t & 1], q);
+            else
+                s_part[t][wave < t ? wave : wave - 1][q][l] = part(acc[t >> 1][t & 1], q);
+        }
+    __syncthreads();
+    const int c = 32 * (wave & 1) + c32, col = n0 + c;
+    if (col >= a.N) return;
+    const float ws = s_ws[c], bb = s_b[c];
+#pragma unroll
+    for (int q = 0; q < 4; ++q) {
+        v4i v = sum[q];
+#pragma unroll
+        for (int o = 0; o < 3; ++o) v += s_part[wave][o][q][l];
+#pragma unroll
+        for (int e = 0; e < 4; ++e) {
+            const int r = 32 * (wave >> 1) + 8 * q + 4 * h + e;
+            float y = (static_cast<float>(v[e]) * s_rs[r]) * ws;
+            if (has_bias) y = y + bb;
+            if (m0 + r < a.M) a.out[static_cast<size_t>(m0 + r) * a.N + col] = y;
+        }
+    }
+}
+
 // The tiled operand order: rows in tiles of T (256 for the activations, 128
 // for the weights), each tile stored stage by stage (64 K bytes), each stage
 // as T rows of 64 bytes with the 16-byte piece p of row r at slot
@@ -415,10 +536,22 @@ hipError_t launch_quantize_rows_tiled(hipStream_t s, const float* x, int m, int 
 }
 
 hipError_t launch_i8_gemm256(hipStream_t s, const int8_t* xt, const float* xs, int m, int k, const int8_t* wt,
-                             const float* ws, int n, const float* bias, float* y) {
+                             const float* ws, int n, const float* bias, float* y, int cu_count) {
     if (!i8_gemm256_supported(m, n, k)) return hipErrorInvalidValue;
     GemmArgs a{xt, xs, wt, ws, bias, y, m, n, k};
     const dim3 grid((m + TM - 1) / TM, (n + TN - 1) / TN);
+    // 64 x 64 blocks where they make one round, two a CU; past it each block's
+    // own reads of 64 rows of both operands cost more than the idle CUs of the
+    // large ones. Large and small, us with the quantize launch, weights cold:
+    // 256 x 3840 x 1280 (rows, columns, K; 240 small blocks) 18.5, 11.9; 512 x
+    // 3840 x 1280 (480) 19.1, 15.9; 768 (720) 20.2, 20.6; 1024 (960) 20.3,
+    // 25.1; 1024 x 1280 x 1280 (320) 19.0, 15.1; 2048 (640) 20.0, 21.6; 1024 x
+    // 1280 x 6848 (320) 70.2, 54.5; 2048 (640) 76.1, 79.8.
+    const int units = ((m + SM - 1) / SM) * ((n + SN - 1) / SN);
+    if (units <= 2 * cu_count) {
+        FOCR_LAUNCH(i8_gemm64_kernel, dim3(kSmXcds * ((units + kSmXcds - 1) / kSmXcds)), dim3(256), 0, s, a);
+        return hipGetLastError();
+    }
     FOCR_LAUNCH(i8_gemm256_kernel, grid, dim3(NTHR), i8_gemm256_lds_bytes(), s, a);
     return hipGetLastError();
 }

@@ -393,8 +393,8 @@ def test_moe_shared_down_inside_down_combine(ctx, h, inter, e, k):
     assert_rel(whole[good], want, 1e-3)
 
 
-@pytest.mark.parametrize("t,e,k,h", [(319, 64, 6, 1280), (320, 64, 6, 1280), (321, 64, 6, 1280), (400, 33, 4, 1264), (513, 16, 3, 272),
-                                     (401, 1, 1, 16)])
+@pytest.mark.parametrize("t,e,k,h", [(319, 64, 6, 1280), (320, 64, 6, 1280), (321, 64, 6, 1280),
+                                     (400, 33, 4, 1264), (513, 16, 3, 272), (401, 1, 1, 16)])
 def test_route_matrix_core_logits(ctx, t, e, k, h):
     """The f64 matrix-core logits at ends of the 16 x 16 tiles and of the waves'
     K shares (1264 and 272 floats: a last line that is partly past the row; 16:

@@ -219,3 +219,20 @@ def test_moe_prefill_i8_narrow_down_blocks(ctx, hidden, inter, si, t):
     st, want = O.moe_prefill_i8(x, idx, gates, *flat, n_e, inter, shared=(si, *[a.reshape(-1) for a in sw]))
     assert st == 0
     assert_rel(out.numpy(), want, 1e-3)
+
+
+@pytest.mark.parametrize("m,k,n,bias", [
+    (256, 64, 64, False),     # one K stage: three of a block's four waves add nothing
+    (256, 1216, 65, True),    # a ring not filled, a column past the block
+    (257, 1280, 127, False),  # the ring exactly full, one row in the last block
+    (319, 1344, 1, True),     # one stage past the ring, one column
+    (320, 2560, 192, False),  # two rings exactly
+    (449, 2624, 640, True),   # and one stage more
+    (448, 320, 4672, False),  # 7 x 73 blocks: 511
+    (512, 320, 4096, False),  # 512
+    (513, 320, 3648, False),  # 9 x 57: 513, past two blocks on each of 256 CUs
+])
+def test_linear_i8_small_blocks_bit_exact(ctx, m, k, n, bias):
+    """64 x 64 blocks with K split over the waves: the i32 sums are exact in any
+    order and the f32 formula is the oracle's, so no difference is allowed."""
+    test_linear_i8_dynamic_bit_exact(ctx, m, k, n, bias)
