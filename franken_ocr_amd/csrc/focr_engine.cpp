@@ -1072,33 +1072,38 @@ int32_t ensure_tiled(focr_hip_ctx* ctx, int8_t** dst, const int8_t* src, size_t 
 
 extern "C" {
 
-// Which kernel an int8 product of m rows takes: the tiled-order GEMMs from 256
-// rows on; below, without a bias, the split-K GEMV in 16-row groups on the
-// upload layout where it is the faster, else 64-row tiles on the fragment-order
-// weight copy. At 256 rows, the GEMV's last size, it took 10.8 us for 1280 x
-// 1280 where the tiled order's 64 x 64 blocks take 6.8; it stays there for a
-// call captured into a graph before the handle has its tiled weights, which
-// cannot be allocated then.
-static bool linear_i8_rows_gemv(focr_hip_ctx* ctx, const focr_hip_qint8* w, size_t m, const float* bias) {
-    if (bias || !gemv_rows_preferred((int)w->n, (int)w->k, (int)m, false)) return false;
-    if (!i8_gemm256_supported((int)m, (int)w->n, (int)w->k)) return true;
-    if (w->w_tiled) return false;
+// Which kernel an int8 product of m rows takes: without a bias, up to 256 rows,
+// the split-K GEMV in 16-row groups on the upload layout where it is the
+// faster, else up to 255 rows 64-row tiles on the fragment-order weight copy;
+// either gives way to the tiled-order GEMMs where i8_gemm_tiled_preferred, and
+// those run everything else. Rows that could go either way stay off the tiled
+// order in a call captured into a graph before the handle has its tiled
+// weights, which cannot be allocated then.
+enum class LinearRoute { kTiled, kGemv, kFragments };
+static LinearRoute linear_i8_route(focr_hip_ctx* ctx, const focr_hip_qint8* w, size_t m, const float* bias) {
+    const int n = (int)w->n, k = (int)w->k;
+    const bool gemv = !bias && gemv_rows_preferred(n, k, (int)m, false);
+    const LinearRoute other = gemv ? LinearRoute::kGemv : LinearRoute::kFragments;
+    if (!i8_gemm_tiled_supported((int)m, n, k)) return other;
+    if (!gemv && m >= 256) return LinearRoute::kTiled;
+    if (!i8_gemm_tiled_preferred((int)m, n, k, ctx->cu_count)) return other;
+    if (w->w_tiled) return LinearRoute::kTiled;
     hipStreamCaptureStatus cap = hipStreamCaptureStatusNone;
-    return hipStreamIsCapturing(ctx->stream, &cap) != hipSuccess || cap != hipStreamCaptureStatusNone;
+    const hipError_t e = hipStreamIsCapturing(ctx->stream, &cap);
+    return e == hipSuccess && cap == hipStreamCaptureStatusNone ? LinearRoute::kTiled : other;
 }
 
 // norm_w (nullable): x is first RMS-normalised with that weight and eps, in
 // the quantize launch; only on the tiled path (the caller checks
 // linear_i8_norm_fusable)
 static bool linear_i8_norm_fusable(focr_hip_ctx* ctx, const focr_hip_qint8* w, size_t m) {
-    return w && !linear_i8_rows_gemv(ctx, w, m, nullptr) && i8_gemm256_supported((int)m, (int)w->n, (int)w->k) &&
-           w->k <= 4096;
+    return w && linear_i8_route(ctx, w, m, nullptr) == LinearRoute::kTiled && w->k <= 4096;
 }
 
 // The activation layout linear_int8_dynamic quantizes x into (row-major, or
 // the tiled order) and its bytes, in the kScrXq slot.
 static bool linear_i8_act_tiled(focr_hip_ctx* ctx, const focr_hip_qint8* w, size_t m, const float* bias) {
-    return !linear_i8_rows_gemv(ctx, w, m, bias) && i8_gemm256_supported((int)m, (int)w->n, (int)w->k);
+    return linear_i8_route(ctx, w, m, bias) == LinearRoute::kTiled;
 }
 static size_t linear_i8_act_bytes(focr_hip_ctx* ctx, const focr_hip_qint8* w, size_t m, const float* bias) {
     return linear_i8_act_tiled(ctx, w, m, bias) ? i8_gemm256_a_bytes((int)m, (int)w->k) : m * w->k;
@@ -1117,7 +1122,8 @@ static int32_t linear_i8_dynamic_impl(focr_hip_ctx* ctx, const focr_hip_qint8* w
                     fmt("linear_int8_dynamic: k %zu is not a multiple of 64 (the matrix-core K stage)", w->k));
     if (norm_w && !linear_i8_norm_fusable(ctx, w, m))
         return fail(FOCR_HIP_E_ARG, "linear_int8_dynamic: the fused norm needs the tiled path");
-    if (linear_i8_rows_gemv(ctx, w, m, bias)) {
+    const LinearRoute route = linear_i8_route(ctx, w, m, bias);
+    if (route == LinearRoute::kGemv) {
         int8_t* xq = static_cast<int8_t*>(ctx->scratch_get(kScrXq, m * w->k));
         float* xs = static_cast<float*>(ctx->scratch_get(kScrXs, m * sizeof(float)));
         if (!xq || !xs) return FOCR_HIP_E_OOM;
@@ -1131,7 +1137,7 @@ static int32_t linear_i8_dynamic_impl(focr_hip_ctx* ctx, const focr_hip_qint8* w
                      "linear_i8 launch");
         return FOCR_HIP_OK;
     }
-    const bool big = i8_gemm256_supported((int)m, (int)w->n, (int)w->k);
+    const bool big = route == LinearRoute::kTiled;
     if (big) {
         if (!w->w_tiled) {
             const size_t bytes = i8_gemm256_b_bytes((int)w->n, (int)w->k);

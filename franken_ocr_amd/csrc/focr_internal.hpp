@@ -585,7 +585,8 @@ hipError_t launch_linear_i8(hipStream_t s, const int8_t* xq, const float* xs, in
 // k_i8gemm.hip — the same product for large row counts: 256 x 128 block
 // tiles, both operands in a tiled order (the activations written so by the
 // quantizer, the weights retiled once). Needs m >= 256 and k a multiple of 64.
-bool i8_gemm256_supported(int m, int n, int k);
+bool i8_gemm_tiled_supported(int m, int n, int k);
+bool i8_gemm_tiled_preferred(int m, int n, int k, int cu_count);  // where another kernel could run too
 size_t i8_gemm256_a_bytes(int m, int k);  // tiled activation buffer
 size_t i8_gemm256_b_bytes(int n, int k);  // tiled weight buffer
 hipError_t launch_i8_gemm256_retile_b(hipStream_t s, const int8_t* w, int n, int k, int8_t* wt);

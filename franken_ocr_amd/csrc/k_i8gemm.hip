@@ -477,12 +477,28 @@ __global__ __launch_bounds__(256) void quantize_rows_tiled_kernel(const float* _
 
 }  // namespace
 
+static long small_blocks(int m, int n) { return static_cast<long>((m + SM - 1) / SM) * ((n + SN - 1) / SN); }
+
 size_t i8_gemm256_lds_bytes() {
     return static_cast<size_t>(NST) * ST_SLOTS * 16 + TM * sizeof(float);
 }
 
-bool i8_gemm256_supported(int m, int n, int k) {
-    return m >= TM && n > 0 && k >= BK && k % BK == 0 && i8_gemm256_lds_bytes() <= max_lds_per_block();
+bool i8_gemm_tiled_supported(int m, int n, int k) {
+    return m > 0 && n > 0 && k >= BK && k % BK == 0 && i8_gemm256_lds_bytes() <= max_lds_per_block();
+}
+
+// Up to 256 rows the split-K GEMV in 16 x 16 groups (or, past its range, 64-row
+// tiles) competes with the 64 x 64 blocks. Its time grows with its groups
+// beyond about three of K = 1280 a CU, theirs hardly. The other kernel and the
+// 64 x 64 blocks, us with the quantize launch, weights cold: 48 rows x 3840
+// columns x 1280 (720 groups) 9.3, 11.1; 64 (960) 12.6, 11.2; 255 20.9, 11.7;
+// 128 x 1280 x 1280 (640) 9.1, 10.1; 160 (800) 11.8, 10.1; 255 13.0, 10.4; 64 x
+// 3584 x 896 (896) 8.6, 10.2; 96 (1344) 11.4, 10.4; 128 x 1280 x 6848 (640)
+// 30.6, 38.9; 200 (1040) 43.4, 38.0; 256 x 640 x 640 (640) 8.0, 9.2.
+bool i8_gemm_tiled_preferred(int m, int n, int k, int cu_count) {
+    const double groups = static_cast<double>((m + 15) / 16) * ((n + 15) / 16), cus = cu_count;
+    return i8_gemm_tiled_supported(m, n, k) && small_blocks(m, n) <= 2l * cu_count && groups > 3 * cus &&
+           groups * k > 3 * cus * 1280;
 }
 
 size_t i8_gemm256_a_bytes(int m, int k) { return static_cast<size_t>((m + TM - 1) / TM) * TM * k; }
@@ -537,7 +553,7 @@ hipError_t launch_quantize_rows_tiled(hipStream_t s, const float* x, int m, int 
 
 hipError_t launch_i8_gemm256(hipStream_t s, const int8_t* xt, const float* xs, int m, int k, const int8_t* wt,
                              const float* ws, int n, const float* bias, float* y, int cu_count) {
-    if (!i8_gemm256_supported(m, n, k)) return hipErrorInvalidValue;
+    if (!i8_gemm_tiled_supported(m, n, k)) return hipErrorInvalidValue;
     GemmArgs a{xt, xs, wt, ws, bias, y, m, n, k};
     const dim3 grid((m + TM - 1) / TM, (n + TN - 1) / TN);
     // 64 x 64 blocks where they make one round, two a CU; past it each block's
@@ -547,9 +563,10 @@ hipError_t launch_i8_gemm256(hipStream_t s, const int8_t* xt, const float* xs, i
     // 3840 x 1280 (480) 19.1, 15.9; 768 (720) 20.2, 20.6; 1024 (960) 20.3,
     // 25.1; 1024 x 1280 x 1280 (320) 19.0, 15.1; 2048 (640) 20.0, 21.6; 1024 x
     // 1280 x 6848 (320) 70.2, 54.5; 2048 (640) 76.1, 79.8.
-    const int units = ((m + SM - 1) / SM) * ((n + SN - 1) / SN);
-    if (units <= 2 * cu_count) {
-        FOCR_LAUNCH(i8_gemm64_kernel, dim3(kSmXcds * ((units + kSmXcds - 1) / kSmXcds)), dim3(256), 0, s, a);
+    const long units = small_blocks(m, n);
+    if (units <= 2l * cu_count) {
+        const unsigned blocks = kSmXcds * static_cast<unsigned>((units + kSmXcds - 1) / kSmXcds);
+        FOCR_LAUNCH(i8_gemm64_kernel, dim3(blocks), dim3(256), 0, s, a);
         return hipGetLastError();
     }
     FOCR_LAUNCH(i8_gemm256_kernel, grid, dim3(NTHR), i8_gemm256_lds_bytes(), s, a);

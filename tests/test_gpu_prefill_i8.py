@@ -231,8 +231,59 @@ def test_moe_prefill_i8_narrow_down_blocks(ctx, hidden, inter, si, t):
     (448, 320, 4672, False),  # 7 x 73 blocks: 511
     (512, 320, 4096, False),  # 512
     (513, 320, 3648, False),  # 9 x 57: 513, past two blocks on each of 256 CUs
+    (144, 1280, 1360, False),  # 765 of the GEMV's groups, three a CU
+    (144, 1280, 1376, False),  # 774, one block row of 16 rows past the second
+    (49, 1280, 3841, False),   # one row block of 49 rows
+    (255, 1792, 1000, True),   # fewer than 256 rows with a bias
 ])
 def test_linear_i8_small_blocks_bit_exact(ctx, m, k, n, bias):
     """64 x 64 blocks with K split over the waves: the i32 sums are exact in any
     order and the f32 formula is the oracle's, so no difference is allowed."""
     test_linear_i8_dynamic_bit_exact(ctx, m, k, n, bias)
+
+
+def _hip():
+    import ctypes
+
+    path = next(ln.split()[-1] for ln in open("/proc/self/maps") if "libamdhip64" in ln)
+    return ctypes.CDLL(path), ctypes
+
+
+@pytest.mark.parametrize("m,k,n", [(256, 1280, 1280), (160, 1280, 1280), (159, 1280, 4096)])
+def test_linear_i8_captured_before_the_tiled_weights(ctx, m, k, n):
+    """A capture cannot allocate the tiled weight copy: a call recorded before
+    the handle has one runs the kernel that needs none (the GEMV; the third
+    shape is past its range and has had its 64-row-tile weights made by a call
+    of few rows), and both give the oracle's bits."""
+    from franken_ocr_amd.engine import QInt8, linear_i8_dynamic
+
+    _say(f"captured linear m={m} k={k} n={n}")
+    hip, ct = _hip()
+    x = synth.f32_normal(synth.seed_of(9900 + m), m * k).reshape(m, k)
+    w = synth.int8_uniform(synth.seed_of(9901), n * k)
+    ws = synth.f32_uniform(synth.seed_of(9902), n, 1e-3, 2e-2)
+    big = QInt8(w, ws, n, k, ctx)
+    dx, dy = ctx.to_device(x), ctx.empty((m, n), np.float32)
+    linear_i8_dynamic(big, dx, dy)  # the scratch, and the tiled route eagerly
+    st, want, _, _ = O.linear_i8_dynamic(x, w, ws, n)
+    assert st == 0 and np.array_equal(dy.numpy(), want)
+    q = QInt8(w, ws, n, k, ctx)
+    if n > 2048:
+        zero = ctx.to_device(np.zeros(n, np.float32))
+        linear_i8_dynamic(q, ctx.to_device(x[:5]), ctx.empty((5, n), np.float32), zero)
+    dz = ctx.to_device(np.zeros((m, n), np.float32))
+    ctx.synchronize()
+    stream, graph, ex = ct.c_void_p(ctx.stream()), ct.c_void_p(), ct.c_void_p()
+    assert hip.hipStreamBeginCapture(stream, 2) == 0  # relaxed
+    try:
+        linear_i8_dynamic(q, dx, dz)
+    finally:
+        rc = hip.hipStreamEndCapture(stream, ct.byref(graph))
+    assert rc == 0
+    assert hip.hipGraphInstantiate(ct.byref(ex), graph, None, None, ct.c_size_t(0)) == 0
+    for _ in range(3):
+        assert hip.hipGraphLaunch(ex, stream) == 0
+        ctx.synchronize()
+        assert np.array_equal(dz.numpy(), want)
+    hip.hipGraphExecDestroy(ex)
+    hip.hipGraphDestroy(graph)
