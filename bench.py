@@ -621,7 +621,7 @@ def cpu_rswa(args, inputs):
 
 
 # ---------------------------------------------------------------------------
-# chunked prefill attention (decoder.rs:1282-1340) on the f32 matrix cores
+# chunked prefill attention (decoder.rs:1282-1340), f32 precision
 # ---------------------------------------------------------------------------
 
 MFMA_F32_PEAK_TFLOPS = 157.3  # dense fp32 MFMA, MI355X

@@ -418,14 +418,14 @@ hipError_t launch_moe_down_combine(hipStream_t s, const MoeDims& d, const uint32
                                    const int* flag, const float* act, const int8_t* wd, const float* sd,
                                    const float* shared_y, const float* resid, float* out, int inter,
                                    const MoeSharedDown* shared = nullptr);
-// k_attn.hip — causal prefill attention on the f32 matrix cores (head_dim
-// 128). Element (row i, head h) of q / out and (key j, head h) of k / v sit at
+// k_attn.hip — causal prefill attention at f32 precision on the bf16 matrix
+// cores (head_dim 128). Element (row i, head h) of q / out and (key j, head h) of k / v sit at
 // base + i * ld + h * hstride (token-major: ld = heads * 128, hstride = 128).
 struct AttnGeom {
     int ldq, hq, ldk, hk, ldv, hv, ldo, ho;
 };
-// Key ranges for a chunk of cs queries over a c1-key prefix: about two
-// blocks per CU, in whole 64-key tiles.
+// Key ranges for a chunk of cs queries over a c1-key prefix, in whole 32-key
+// tiles: the length with the least estimated time.
 int attn_pick_splits(int cs, int c1, int heads, int cu_count, int* split_len);
 size_t attn_partials_bytes(int cs, int heads, int nsplit);
 // qo (nullable): where the split merge may write the context rows quantized

@@ -358,7 +358,7 @@ int32_t focr_hip_moe_prefill_i8(focr_hip_ctx* ctx, const focr_hip_moe_layer* lay
                                 size_t t, const uint32_t* idx, const float* gates,
                                 int32_t with_shared, float* out, int32_t check_idx);
 
-/* ---- prefill attention on the f32 matrix cores -----------------------------
+/* ---- prefill attention on the matrix cores ---------------------------------
  * decoder.rs:1282-1340 chunk_prefill_attention: the cs = c1 - c0 queries
  * q_chunk [cs, num_heads*head_dim] (global positions [c0, c1), RoPE applied)
  * attend over the prefix k_prefix / v_prefix [c1, num_heads*head_dim] under
@@ -367,8 +367,8 @@ int32_t focr_hip_moe_prefill_i8(focr_hip_ctx* ctx, const focr_hip_moe_layer* lay
  * h*head_dim ..). E_SHAPE with the reference's message when c0 > c1 or
  * c0 + cs != c1 ("chunk_prefill_attention: chunk [c0, c0+cs) of cs rows does
  * not fit prefix c1"); head_dim must be 128 (E_SHAPE otherwise). f32
- * throughout (f32 MFMAs); agrees with the reference's f32 attention to
- * rounding (rel 1e-4). Device pointers. */
+ * precision (operands as three-term bf16 splits, f32 sums); agrees with the
+ * reference's f32 attention to rounding (rel 1e-4). Device pointers. */
 int32_t focr_hip_chunk_prefill_attention(focr_hip_ctx* ctx, const float* q_chunk, size_t cs,
                                          const float* k_prefix, const float* v_prefix, size_t c1,
                                          size_t num_heads, size_t head_dim, size_t c0, float* out);
