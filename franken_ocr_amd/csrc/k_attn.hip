@@ -454,6 +454,264 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(kBlocksPerC
     }
 }
 
+// Combine lane l's value with lanes l ^ 16, l ^ 32, l ^ 48 (the four 16-lane
+// rows): gfx950's v_permlane16_swap / v_permlane32_swap of a value with itself
+// put both partners of an xor-16 (xor-32) pair in each lane (VALU; the
+// shuffle form went through ds_bpermute at LDS latency). The pairs combine as
+// the xor butterfly did: (r0 op r1) op (r2 op r3) in every lane.
+__device__ __forceinline__ float perm16_lo(float v, float& hi) {
+    const auto r = __builtin_amdgcn_permlane16_swap(__float_as_uint(v), __float_as_uint(v), false, false);
+    hi = __uint_as_float(r[1]);
+    return __uint_as_float(r[0]);
+}
+__device__ __forceinline__ float perm32_lo(float v, float& hi) {
+    const auto r = __builtin_amdgcn_permlane32_swap(__float_as_uint(v), __float_as_uint(v), false, false);
+    hi = __uint_as_float(r[1]);
+    return __uint_as_float(r[0]);
+}
+__device__ __forceinline__ float wave16_max(float v) {
+    float b;
+    const float a = perm16_lo(v, b);
+    v = fmaxf(a, b);
+    const float c = perm32_lo(v, b);
+    return fmaxf(c, b);
+}
+__device__ __forceinline__ float wave16_sum(float v) {
+    float b;
+    const float a = perm16_lo(v, b);
+    v = a + b;
+    const float c = perm32_lo(v, b);
+    return c + b;
+}
+
+// ---- few rows and keys: f32 matrix cores ------------------------------------
+// A call of a few key ranges is one chain of latencies: query rows, first tile,
+// its products, output, merge. The kernel above puts 128 query rows, their
+// splits and a pass through LDS for the output into that chain; this one has
+// 64 rows a block, 16 a wave, and exact f32 products on v_mfma_f32_16x16x4, so
+// its chain is shorter and its rate an eighth. Whole calls, this kernel and the
+// one above, us: 16 rows 5.3, 8.1; 64 rows 10.1, 11.8; 128 rows 11.4, 18.6; 192
+// rows 13.3, 15.1; 64 rows after 448 keys 12.6, 16.3; 128 after 128 12.8, 15.3,
+// after 384 17.9, 18.7. Past that it loses: 256 rows 17.0, 16.4; 16 after 500
+// 16.8, 14.9; 256 after 256 22.9, 20.7; 64 after 960 32.5, 19.7.
+// Scores come as S^T = K Q^T (A = 16 keys x 4 dims from LDS, B = 4 dims x 16
+// query rows in registers), so lane (g, j) holds row j's scores of keys 16 n +
+// 4 g + r, the B operand of the P V product; dims in the order 8 (4 g + r') + m
+// leave each lane 32 consecutive dims of its row. Ranges and partials are those
+// of the kernel above, so the merge is shared.
+constexpr int kSmRT = 64;                  // query rows per block
+constexpr int kSmBlocksPerCu = 3;          // residency (LDS 34 KB, 143 VGPRs)
+constexpr int kLdsRow = kD + 4;            // padded LDS row (floats)
+constexpr int kSub = kKT / 16;             // 16-key MFMA subtiles per tile
+constexpr int kPieces = kKT * kD / 4 / 256;  // float4 of one matrix per thread and tile
+
+__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(kSmBlocksPerCu))) void attn_prefill_small_kernel(
+    const AttnArgs a) {
+    extern __shared__ float4 lds_kv4[];  // K tile then V tile, [kKT][kLdsRow] floats each
+    float* lk = reinterpret_cast<float*>(lds_kv4);
+    float* lv = lk + kKT * kLdsRow;
+    const int wave = threadIdx.x >> 6;
+    const int lane = threadIdx.x & 63;
+    const int g = lane >> 4, j = lane & 15;
+    const int h = blockIdx.y;
+    const int split = blockIdx.z;
+    const int row0 = blockIdx.x * 64;            // block's first chunk row
+    const int wrow = row0 + wave * 16 + j;        // this lane's chunk row
+    const int qrow = wrow < a.cs ? wrow : a.cs - 1;
+    const int t = a.c0 + wrow;                    // its global position
+    // keys this block needs: [0, min(c1, c0 + row0 + 64)), this split's part
+    const int kmax = min(a.c1, a.c0 + row0 + 64);
+    const int ks = split * a.split_len;
+    const int ke = min(ks + a.split_len, kmax);
+    // a range past these 64 rows' last key; the merge goes by tiles of kRT
+    // rows, so it finds an empty range; block-uniform
+    if (ks >= ke) {
+        if (wrow < a.cs && g == 0 && ks < min(a.c1, a.c0 + (row0 / kRT + 1) * kRT))
+            *reinterpret_cast<float2*>(
+                a.part_ml + ((static_cast<size_t>(split) * a.heads + h) * a.cs + wrow) * 2) =
+                make_float2(-INFINITY, 0.0f);
+        return;
+    }
+
+    // Q fragment: qf[s] = q[row j][32g + s], s = 0..31
+    float qf[32];
+    {
+        const float4* qp = reinterpret_cast<const float4*>(a.q + static_cast<size_t>(qrow) * a.ldq +
+                                                           static_cast<size_t>(h) * a.hq + 32 * g);
+#pragma unroll
+        for (int u = 0; u < 8; ++u) {
+            const v4f x = *reinterpret_cast<const v4f*>(qp + u);
+            qf[4 * u] = x.x;
+            qf[4 * u + 1] = x.y;
+            qf[4 * u + 2] = x.z;
+            qf[4 * u + 3] = x.w;
+        }
+    }
+    v4f oacc[8];
+#pragma unroll
+    for (int m = 0; m < 8; ++m) oacc[m] = v4f{0.0f, 0.0f, 0.0f, 0.0f};
+    float m_run = -INFINITY, l_run = 0.0f;
+
+    // tile loads: 32 keys x 128 floats = 1024 float4 per matrix, 4 per thread
+    const int c4 = threadIdx.x & 31;  // float4 column
+    const int r8 = threadIdx.x >> 5;  // 8 rows per pass
+    const float* kh = a.k + static_cast<size_t>(h) * a.hk + 4 * c4;
+    const float* vh = a.v + static_cast<size_t>(h) * a.hv + 4 * c4;
+    // Tile loads of keys kb .. kb + kKT - 1 (rows clamped into the prefix; a
+    // row past the range end is never used) and their LDS stores.
+    v4f pk[kPieces], pv[kPieces];
+    auto load_tile = [&](int kb) {
+#pragma unroll
+        for (int p = 0; p < kPieces; ++p) {
+            int key = kb + r8 + 8 * p;
+            key = key < a.c1 ? key : a.c1 - 1;
+            pk[p] = *reinterpret_cast<const v4f*>(kh + static_cast<size_t>(key) * a.ldk);
+            pv[p] = *reinterpret_cast<const v4f*>(vh + static_cast<size_t>(key) * a.ldv);
+        }
+    };
+    auto store_tile = [&]() {
+#pragma unroll
+        for (int p = 0; p < kPieces; ++p) {
+            *reinterpret_cast<v4f*>(lk + (r8 + 8 * p) * kLdsRow + 4 * c4) = pk[p];
+            *reinterpret_cast<v4f*>(lv + (r8 + 8 * p) * kLdsRow + 4 * c4) = pv[p];
+        }
+    };
+    if (ks < ke) {
+        load_tile(ks);
+        store_tile();
+    }
+    // every load so far (the Q fragment too) complete on every path into
+    // the loop, so the loop's first MFMAs wait for none of the tile loads
+    // issued inside it (vmcnt(0): the counter drains in issue order)
+    __builtin_amdgcn_s_waitcnt(0x0F70);
+    __syncthreads();
+    // Each iteration issues the next tile's loads first, consumes the
+    // current tile from LDS while they are in flight, then (after every wave
+    // has read it) stores the next tile over it. The loads are consumed in
+    // the iteration that issues them: a load carried into the next iteration
+    // was folded with the one before the loop into a single load at the top
+    // of the loop, which waited out a full memory round trip on every tile.
+    for (int kb = ks; kb < ke; kb += kKT) {
+        const bool more = kb + kKT < ke;
+        if (more) load_tile(kb + kKT);
+        __builtin_amdgcn_sched_barrier(0);  // the loads go out before the tile's MFMAs
+
+        // S^T for the subtiles of 16 keys; each score dot runs as two
+        // 16-step MFMA chains (dims 32g + 16h + [0, 16), h = 0, 1) added at
+        // the end, halving the f32 accumulation chain of the 128-term dot.
+        // The 2 * kSub chains advance together: each step reads their four
+        // dims of K (one 16-byte LDS read per chain) and issues one MFMA per
+        // chain and dim, so a chain's dependent MFMAs interleave with the
+        // other chains' (each chain's own order is unchanged: u, then dim).
+        v4f sc[kSub][2];
+#pragma unroll
+        for (int n = 0; n < kSub; ++n) sc[n][0] = sc[n][1] = v4f{0.0f, 0.0f, 0.0f, 0.0f};
+#pragma unroll
+        for (int u2 = 0; u2 < 4; ++u2) {
+            v4f kf[kSub][2];
+#pragma unroll
+            for (int n = 0; n < kSub; ++n)
+#pragma unroll
+                for (int hh = 0; hh < 2; ++hh)
+                    kf[n][hh] = *reinterpret_cast<const v4f*>(lk + (16 * n + j) * kLdsRow + 32 * g + 16 * hh + 4 * u2);
+#pragma unroll
+            for (int c = 0; c < 4; ++c)
+#pragma unroll
+                for (int n = 0; n < kSub; ++n)
+#pragma unroll
+                    for (int hh = 0; hh < 2; ++hh)
+                        sc[n][hh] = __builtin_amdgcn_mfma_f32_16x16x4f32(kf[n][hh][c], qf[16 * hh + 4 * u2 + c],
+                                                                         sc[n][hh], 0, 0, 0);
+        }
+        v4f sacc[kSub];
+#pragma unroll
+        for (int n = 0; n < kSub; ++n) sacc[n] = sc[n][0] + sc[n][1];
+        // scale, causal / range mask, online softmax (row j over 4 lanes)
+        float pr[kSub][4];
+        float tmax = -INFINITY;
+#pragma unroll
+        for (int n = 0; n < kSub; ++n)
+#pragma unroll
+            for (int r = 0; r < 4; ++r) {
+                const int key = kb + 16 * n + 4 * g + r;
+                const float sv = sacc[n][r] * a.scale;
+                const bool ok = key <= t && key < ke;
+                pr[n][r] = ok ? sv : -INFINITY;
+                tmax = fmaxf(tmax, pr[n][r]);
+            }
+        tmax = wave16_max(tmax);
+        const float m_new = fmaxf(m_run, tmax);
+        const float corr = m_run == -INFINITY ? 0.0f : __builtin_amdgcn_exp2f(m_run - m_new);
+        float tsum = 0.0f;
+#pragma unroll
+        for (int n = 0; n < kSub; ++n)
+#pragma unroll
+            for (int r = 0; r < 4; ++r) {
+                const float p = pr[n][r] == -INFINITY ? 0.0f : __builtin_amdgcn_exp2f(pr[n][r] - m_new);
+                pr[n][r] = p;
+                tsum += p;
+            }
+        tsum = wave16_sum(tsum);
+        l_run = l_run * corr + tsum;
+        m_run = m_new;
+        // the running output rescaled to the new max, then this tile's
+        // V^T . P^T accumulated into it (step (n, r) is key kb + 16n + 4g + r)
+#pragma unroll
+        for (int m = 0; m < 8; ++m) oacc[m] = oacc[m] * corr;
+#pragma unroll
+        for (int n = 0; n < kSub; ++n)
+#pragma unroll
+            for (int r = 0; r < 4; ++r) {
+                const float* vr = lv + (16 * n + 4 * g + r) * kLdsRow + 8 * j;
+                const v4f v0 = *reinterpret_cast<const v4f*>(vr);
+                const v4f v1 = *reinterpret_cast<const v4f*>(vr + 4);
+                const float b = pr[n][r];
+                oacc[0] = __builtin_amdgcn_mfma_f32_16x16x4f32(v0.x, b, oacc[0], 0, 0, 0);
+                oacc[1] = __builtin_amdgcn_mfma_f32_16x16x4f32(v0.y, b, oacc[1], 0, 0, 0);
+                oacc[2] = __builtin_amdgcn_mfma_f32_16x16x4f32(v0.z, b, oacc[2], 0, 0, 0);
+                oacc[3] = __builtin_amdgcn_mfma_f32_16x16x4f32(v0.w, b, oacc[3], 0, 0, 0);
+                oacc[4] = __builtin_amdgcn_mfma_f32_16x16x4f32(v1.x, b, oacc[4], 0, 0, 0);
+                oacc[5] = __builtin_amdgcn_mfma_f32_16x16x4f32(v1.y, b, oacc[5], 0, 0, 0);
+                oacc[6] = __builtin_amdgcn_mfma_f32_16x16x4f32(v1.z, b, oacc[6], 0, 0, 0);
+                oacc[7] = __builtin_amdgcn_mfma_f32_16x16x4f32(v1.w, b, oacc[7], 0, 0, 0);
+            }
+        if (more) {  // block-uniform
+            __syncthreads();  // every wave is done with this tile
+            store_tile();
+            __syncthreads();
+        }
+    }
+    if (wrow >= a.cs) return;
+    // lane (g, j) holds O[row j][32g + 8r' + m] in oacc[m][r']
+    if (a.nsplit == 1) {
+        const float inv = 1.0f / l_run;
+        float* op = a.out + static_cast<size_t>(wrow) * a.ldo + static_cast<size_t>(h) * a.ho + 32 * g;
+#pragma unroll
+        for (int rr = 0; rr < 4; ++rr) {
+            float4 x0, x1;
+            x0.x = oacc[0][rr] * inv;
+            x0.y = oacc[1][rr] * inv;
+            x0.z = oacc[2][rr] * inv;
+            x0.w = oacc[3][rr] * inv;
+            x1.x = oacc[4][rr] * inv;
+            x1.y = oacc[5][rr] * inv;
+            x1.z = oacc[6][rr] * inv;
+            x1.w = oacc[7][rr] * inv;
+            *reinterpret_cast<float4*>(op + 8 * rr) = x0;
+            *reinterpret_cast<float4*>(op + 8 * rr + 4) = x1;
+        }
+        return;
+    }
+    const size_t pidx = (static_cast<size_t>(split) * a.heads + h) * a.cs + wrow;
+    float* op = a.part_o + pidx * kD + 32 * g;
+#pragma unroll
+    for (int rr = 0; rr < 4; ++rr) {
+        *reinterpret_cast<float4*>(op + 8 * rr) = make_float4(oacc[0][rr], oacc[1][rr], oacc[2][rr], oacc[3][rr]);
+        *reinterpret_cast<float4*>(op + 8 * rr + 4) = make_float4(oacc[4][rr], oacc[5][rr], oacc[6][rr], oacc[7][rr]);
+    }
+    if (g == 0) *reinterpret_cast<float2*>(a.part_ml + pidx * 2) = make_float2(m_run, l_run);
+}
+
 // Fold the key ranges: out = sum_s 2^(m_s - M) O_s / sum_s 2^(m_s - M) l_s,
 // M = max_s m_s, the maxima in base-2 units (a range with no key of the row
 // has m = -inf, l = 0, O = 0). Only the ranges below the row tile's last key
@@ -599,7 +857,23 @@ size_t attn_partials_bytes(int cs, int heads, int nsplit) {
     return static_cast<size_t>(nsplit) * heads * cs * (kD + 2) * sizeof(float);
 }
 
+// Rows and keys for which attn_prefill_small_kernel is taken (measured beside it)
+static bool attn_small(int cs, int c1) { return cs <= 192 && c1 <= 512 && cs * c1 <= 65536; }
+
 int attn_pick_splits(int cs, int c1, int heads, int cu_count, int* split_len) {
+    if (attn_small(cs, c1)) {
+        // the shortest ranges whose blocks are resident at once
+        const long long slots = static_cast<long long>(kSmBlocksPerCu) * (cu_count > 0 ? cu_count : 1);
+        int per = 1;
+        for (;; ++per) {
+            long long blocks = 0;
+            for (int r = 0; r < cs; r += kSmRT)
+                blocks += ((min(c1, c1 - cs + r + kSmRT) + kKT - 1) / kKT + per - 1) / per;
+            if (blocks * heads <= slots || per * kKT >= c1) break;
+        }
+        *split_len = per * kKT;
+        return (c1 + *split_len - 1) / *split_len;
+    }
     // Row tile i (kRT rows) needs the tiles of keys [0, min(c1, c0 + kRT (i + 1))):
     // ranges of `per` tiles give sum over i of ceil(n_i / per) blocks per
     // head. The length taken is the one with the least estimated time (us),
@@ -646,9 +920,14 @@ hipError_t launch_attn_prefill(hipStream_t s, const AttnGeom& gm, const float* q
         a.part_o = part;
         a.part_ml = part + static_cast<size_t>(nsplit) * heads * cs * kD;
     }
-    int ranges = 0;
-    for (int r = 0; r < cs; r += kRT) ranges += (min(c1, c0 + r + kRT) + split_len - 1) / split_len;
-    FOCR_LAUNCH(attn_prefill_kernel, dim3(heads, ranges), dim3(256), 0, s, a);
+    if (attn_small(cs, c1)) {
+        FOCR_LAUNCH(attn_prefill_small_kernel, dim3((cs + kSmRT - 1) / kSmRT, heads, nsplit), dim3(256),
+                    2 * kKT * kLdsRow * sizeof(float), s, a);
+    } else {
+        int ranges = 0;
+        for (int r = 0; r < cs; r += kRT) ranges += (min(c1, c0 + r + kRT) + split_len - 1) / split_len;
+        FOCR_LAUNCH(attn_prefill_kernel, dim3(heads, ranges), dim3(256), 0, s, a);
+    }
     hipError_t e = hipGetLastError();
     if (qo) qo->done = false;
     if (e != hipSuccess || nsplit == 1) return e;
