@@ -40,7 +40,8 @@ def _close(got, want):
     assert err.max() <= 1e-4, float(err.max())
 
 
-@pytest.mark.parametrize("rows,c0", [(31, 0), (33, 1), (96, 31), (127, 33), (128, 0), (129, 640), (1, 2047), (260, 95)])
+@pytest.mark.parametrize("rows,c0", [(31, 0), (33, 1), (96, 31), (127, 33), (128, 0), (129, 640), (1, 2047), (260, 95),
+                                     (192, 149), (193, 0), (64, 448), (64, 449), (1, 511), (1, 512), (66, 300)])
 def test_row_and_key_tile_edges(ctx, rows, c0):
     q, k, v = _qkv(4100 + rows, rows, c0)
     st, want = O.chunk_prefill_attention(q, k, v, NH, D, c0)
