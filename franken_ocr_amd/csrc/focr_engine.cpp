@@ -1660,12 +1660,13 @@ static int32_t decoder_layer_step_impl(focr_hip_ctx* ctx, const focr_hip_decoder
         return moe_decode_impl(ctx, L->moe, x, B, 0, 1.0f, L->moe->swg ? 1 : 0, x, route_idx, nullptr, check_route,
                                h, false, &rn);
     }
-    // dense (layer 0) in three launches where the shapes allow: the residual,
-    // the post-attention norm, quantize, the gate and up GEMVs and SiLU(g) * u
+    // dense (layer 0) in three launches where the shapes allow and x can be
+    // read 16 bytes a lane (x is the caller's and may start anywhere; the
+    // separate kernels below take it so): the residual, the post-attention norm, quantize, the gate and up GEMVs and SiLU(g) * u
     // in one (h = x + attn stored by it); quantize_row_i8 of act; the down
     // GEMV with the residual add in its epilogue (x = h + down(act))
     const int cu = ctx->cu_count > 0 ? ctx->cu_count : 256;
-    if (!L->moe && L->gate_up_w && H % 64 == 0 && H <= 1280 && I % 64 == 0 && I <= 8192 &&
+    if (!L->moe && L->gate_up_w && aligned16(x) && H % 64 == 0 && H <= 1280 && I % 64 == 0 && I <= 8192 &&
         (I + 15) / 16 < static_cast<size_t>(4 * cu) && (H + 15) / 16 < static_cast<size_t>(4 * cu)) {
         float* act = reinterpret_cast<float*>(take(B * I * 4));
         int8_t* aq = reinterpret_cast<int8_t*>(take(B * I));

@@ -99,7 +99,7 @@ def _prefill(ctx, B, seed):
 
 
 # moe 20: a second 16-row qkv pass; dense 2 / 8 (its stream limit): the
-# three-launch dense MLP; dense 1: the separate kernels it replaces
+# three-launch dense MLP, dense 1 at one row
 @pytest.mark.parametrize("kind,B", [("moe", 4), ("dense", 2), ("moe", 20), ("dense", 8), ("dense", 1)])
 def test_decoder_layer_steps_match_oracle(ctx, kind, B):
     _say(f"{kind} layer, {B} streams, 3 steps")
@@ -118,6 +118,30 @@ def test_decoder_layer_steps_match_oracle(ctx, kind, B):
         assert_rel(got, want, 1e-3)
         _say(f"step {step}: max |got - want| {np.abs(got - want).max():.3e}")
         want = got  # continue from the device's state (both rings hold the same steps)
+
+
+@pytest.mark.parametrize("kind,B", [("dense", 1), ("dense", 2), ("dense", 12), ("moe", 1), ("moe", 3)])
+def test_decoder_layer_takes_rows_that_start_anywhere(ctx, kind, B):
+    """x four bytes past a 16-byte boundary (a view into a larger buffer): the
+    forms that read rows 16 bytes a lane give way to the separate kernels, and
+    the step is the aligned one's, its cursors too, over two steps."""
+    _say(f"{kind} layer, {B} streams, x at 4 bytes past a boundary")
+    lw = _weights(14000 if kind == "moe" else 14500, None if kind == "moe" else 6848)
+    layer = _gpu_layer(ctx, lw)
+    x = synth.f32_normal(synth.seed_of(14800), B * H)
+    pos = np.array([G + s for s in range(B)], np.uint32)
+    outs = []
+    for skip in (0, 1):
+        cache, _, _ = _prefill(ctx, B, 14600)
+        buf = ctx.to_device(np.concatenate([np.full(skip, 7.0, np.float32), x]).reshape(-1, 1))
+        rows = buf.view_rows(skip, skip + B * H)
+        assert rows.ptr % 16 == 4 * skip
+        for step in range(2):
+            layer.step(cache, pos + step, rows, check_route=False)
+        assert [cache.state(s) for s in range(B)] == [(G, 2, 2)] * B
+        outs.append(rows.numpy())
+        cache.free()
+    assert_rel(outs[1], outs[0], 1e-3)
 
 
 @pytest.mark.parametrize("kind,B", [("moe", 40), ("dense", 12)])
