@@ -1,8 +1,10 @@
 """The prefill attention's edges on the GPU: the row tiles (32 per wave, 128
 per block), the 32-key tiles and the key ranges, against the float64 oracle
 (rel 1e-4 on the floored metric, the attention tolerance); and values that the
-kernel's three-term bf16 split does not cover (infinities, magnitudes whose
-bf16 is infinite) or covers at the end of its range."""
+large form's three-term bf16 split does not cover (infinities, magnitudes whose
+bf16 is infinite) or covers at the end of its range. Up to 192 rows and 512
+keys a call takes the small form, which has f32 products and no split: each of
+these tests runs on both, 260 rows after 95 and 300 after 700 being past it."""
 
 from __future__ import annotations
 
@@ -49,23 +51,29 @@ def test_row_and_key_tile_edges(ctx, rows, c0):
     _close(_run(ctx, q, k, v, c0), want)
 
 
-@pytest.mark.parametrize("scale", [1.0e34, 1.0e-34])
-def test_values_at_the_ends_of_the_range(ctx, scale):
-    # 1e-34 v: the split's third terms are subnormal. 1e34 v with two values
-    # whose bf16 is infinite: the unnormalised sums (at most 3.399e38 + 330 *
-    # 5e34 per value column) stay below f32's 3.403e38.
-    q, k, v = _qkv(4300, 130, 200)
+@pytest.mark.parametrize("rows,c0,scale", [(130, 200, 1.0e34), (130, 200, 1.0e-34), (260, 95, 1.0e31),
+                                           (260, 95, 1.0e-34), (300, 700, 1.0e31), (300, 700, 1.0e-34)])
+def test_values_at_the_ends_of_the_range(ctx, rows, c0, scale):
+    # 1e-34 v: the split's third terms are subnormal. Large v with two values
+    # whose bf16 is infinite: at 1e31 the unnormalised sums are at most
+    # 3.399e38 + 1000 * 6e31, below f32's 3.403e38 (at 1e34 they are because
+    # no row gives either value a probability near 1)
+    q, k, v = _qkv(4300, rows, c0)
     v = (v * np.float32(scale)).astype(np.float32)
     if scale > 1:
         v[7, 5], v[150, 700] = 3.399e38, -3.399e38
-    st, want = O.chunk_prefill_attention(q, k, v, NH, D, 200)
+    st, want = O.chunk_prefill_attention(q, k, v, NH, D, c0)
     assert st == 0 and np.isfinite(want).all()
-    _close(_run(ctx, q, k, v, 200), want)
+    _close(_run(ctx, q, k, v, c0), want)
 
 
+# three keys a tile apart: in ranges of two tiles or more, one of them at the
+# least lies past its range's first tile
 @pytest.mark.parametrize("bad", [np.inf, -np.inf, np.nan])
-def test_an_infinite_or_nan_value_reaches_the_rows_that_see_it(ctx, bad):
-    rows, c0, key, col = 140, 70, 100, 3 * D + 9
+@pytest.mark.parametrize("rows,c0,key", [(140, 70, 100), (260, 95, 100), (260, 95, 132), (260, 95, 164),
+                                         (300, 700, 610), (300, 700, 642), (300, 700, 990)])
+def test_an_infinite_or_nan_value_reaches_the_rows_that_see_it(ctx, rows, c0, key, bad):
+    col = 3 * D + 9
     q, k, v = _qkv(4400, rows, c0)
     st, want = O.chunk_prefill_attention(q, k, v, NH, D, c0)
     v[key, col] = bad
@@ -76,8 +84,9 @@ def test_an_infinite_or_nan_value_reaches_the_rows_that_see_it(ctx, bad):
     np.testing.assert_array_equal(got[sees, col], np.full(sees.sum(), bad, np.float32))
 
 
-def test_a_key_of_minus_infinite_score_is_not_seen(ctx):
-    rows, c0, key = 40, 60, 30
+@pytest.mark.parametrize("rows,c0,key", [(40, 60, 30), (260, 95, 30), (260, 95, 62), (260, 95, 94), (300, 700, 610),
+                                         (300, 700, 642)])
+def test_a_key_of_minus_infinite_score_is_not_seen(ctx, rows, c0, key):
     q, k, v = _qkv(4500, rows, c0)
     q[:, :D] = np.abs(q[:, :D]) + 0.5
     k[key, 4] = -np.inf  # head 0's score of that key is -inf for every row
@@ -85,3 +94,29 @@ def test_a_key_of_minus_infinite_score_is_not_seen(ctx):
     st, want = O.chunk_prefill_attention(q, k2, v2, NH, D, c0 - 1)
     assert st == 0
     _close(_run(ctx, q, k, v, c0)[:, :D], want[:, :D])
+
+
+@pytest.mark.parametrize("rows,c0", [(40, 60), (260, 95), (300, 700)])
+def test_a_finite_key_whose_bf16_is_infinite(ctx, rows, c0):
+    q, k, v = _qkv(4600, rows, c0)
+    q[:, 4] = 0.0  # head 0 does not look at the dim
+    st, want = O.chunk_prefill_attention(q, k, v, NH, D, c0)
+    assert st == 0
+    k[c0 + 20, 4], k[5, 4] = 3.399e38, -3.399e38
+    _close(_run(ctx, q, k, v, c0), want)
+
+
+@pytest.mark.parametrize("bad", [np.inf, np.nan])
+@pytest.mark.parametrize("rows,c0", [(40, 60), (260, 95), (300, 700)])
+def test_a_query_that_is_not_finite_stays_in_its_row(ctx, rows, c0, bad):
+    q, k, v = _qkv(4700, rows, c0)
+    st, want = O.chunk_prefill_attention(q, k, v, NH, D, c0)
+    assert st == 0
+    row = rows - 7
+    q[row, D + 3] = bad  # head 1
+    got = _run(ctx, q, k, v, c0)
+    assert np.isnan(got[row, D:2 * D]).all()
+    keep = np.ones_like(got, bool)
+    keep[row, D:2 * D] = False
+    want = np.where(keep, want, 0.0)
+    _close(np.where(keep, got, 0.0), want)
