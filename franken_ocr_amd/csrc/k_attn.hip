@@ -118,6 +118,19 @@ __device__ __forceinline__ float chk_terms(float chk, uint32_t w1) {
     return __builtin_amdgcn_fdot2_f32_bf16(__builtin_bit_cast(v2bf, w1), __builtin_bit_cast(v2bf, 0u), chk, false);
 }
 
+// Below kMinSplit the third term runs out of bf16's range (its last bit is at
+// 2^-133; the least term of 2^-100 is at 2^-123, still a normal number), so
+// nonzero values below it have no split either. low_abs keeps the least
+// magnitude that a thread stages, a v_min3 a pair; only where that is small is
+// it seen whether the value is an ordinary zero. (An exact test of every value
+// is three instructions a pair.)
+constexpr float kMinSplit = 0x1p-100f;
+__device__ __forceinline__ float low_abs(float low, float a, float b) {
+    asm("v_min3_f32 %0, |%1|, |%2|, %0" : "+v"(low) : "v"(a), "v"(b));
+    return low;
+}
+__device__ __forceinline__ bool too_low(float x) { return x != 0.0f && fabsf(x) < kMinSplit; }
+
 struct Split8 {
     v4u w[3];  // terms 1, 2, 3 of eight values
     __device__ __forceinline__ void pair(int i, float a, float b, float& chk) {
@@ -279,7 +292,14 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(kBlocksPerC
                                                           4 * a.ldv * min(vkey0 + (i & 3) + 8 * (i >> 2), last), 0));
     };
     auto store_k = [&]() {
-        float chk = 0.0f;
+        float chk = 0.0f, low = INFINITY;
+#pragma unroll
+        for (int p = 0; p < 4; ++p) low = low_abs(low_abs(low, pk[p].x, pk[p].y), pk[p].z, pk[p].w);
+        if (low < kMinSplit) {
+#pragma unroll
+            for (int p = 0; p < 4; ++p)
+                if (too_low(pk[p].x) || too_low(pk[p].y) || too_low(pk[p].z) || too_low(pk[p].w)) chk = NAN;
+        }
 #pragma unroll
         for (int p = 0; p < 2; ++p) {
             Split8 s;
@@ -292,7 +312,14 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(kBlocksPerC
         if (chk != chk) bad[0] = 1;
     };
     auto store_v = [&]() {
-        float chk = 0.0f;
+        float chk = 0.0f, low = INFINITY;
+#pragma unroll
+        for (int i = 0; i < 8; ++i) low = low_abs(low, pv[i].x, pv[i].y);
+        if (low < kMinSplit) {
+#pragma unroll
+            for (int i = 0; i < 8; ++i)
+                if (too_low(pv[i].x) || too_low(pv[i].y)) chk = NAN;
+        }
 #pragma unroll
         for (int e = 0; e < 2; ++e) {
             Split8 s;
@@ -318,15 +345,24 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(kBlocksPerC
         rows[(2 * i + hf) * kORow + j] =
             *reinterpret_cast<const v4u*>(qh + static_cast<size_t>(min(wrow0 + 2 * i + hf, a.cs - 1)) * a.ldq);
     Split8 qf[8];
-    float qchk = 0.0f;
+    float qchk = 0.0f, qlow = INFINITY;
 #pragma unroll
     for (int s = 0; s < 8; ++s) {
         const v4f x0 = __builtin_bit_cast(v4f, rows[j * kORow + 4 * s + 2 * hf]);
         const v4f x1 = __builtin_bit_cast(v4f, rows[j * kORow + 4 * s + 2 * hf + 1]);
+        qlow = low_abs(low_abs(qlow, x0.x, x0.y), x0.z, x0.w);
+        qlow = low_abs(low_abs(qlow, x1.x, x1.y), x1.z, x1.w);
         qf[s].pair(0, x0.x, x0.y, qchk);
         qf[s].pair(1, x0.z, x0.w, qchk);
         qf[s].pair(2, x1.x, x1.y, qchk);
         qf[s].pair(3, x1.z, x1.w, qchk);
+    }
+    if (qlow < kMinSplit) {
+#pragma unroll 1
+        for (int i = 0; i < kD; i += 4) {
+            const v4f x = __builtin_bit_cast(v4f, rows[j * kORow + i / 4]);
+            if (too_low(x.x) || too_low(x.y) || too_low(x.z) || too_low(x.w)) qchk = NAN;
+        }
     }
     // the third terms of steps 0 .. kQLds - 1 stay in LDS (all in registers spills)
     v4u* lqw = lv + 3 * kVTerm + wave * kQLds * 64 + lane;

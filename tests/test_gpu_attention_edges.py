@@ -120,3 +120,17 @@ def test_a_query_that_is_not_finite_stays_in_its_row(ctx, rows, c0, bad):
     keep[row, D:2 * D] = False
     want = np.where(keep, want, 0.0)
     _close(np.where(keep, got, 0.0), want)
+
+
+@pytest.mark.parametrize("rows,c0", [(40, 60), (260, 95), (300, 700)])
+@pytest.mark.parametrize("sq,sk,sv", [(1.0, 1.0, 1e-35), (1.0, 1.0, 1e-37), (1e-36, 1e36, 1.0), (1e36, 1e-36, 1.0)])
+def test_values_too_small_for_three_bf16_terms(ctx, rows, c0, sq, sk, sv):
+    """Magnitudes whose third bf16 term has no bits left (f32 products keep
+    them, subnormal results included), among zeros, which have a split."""
+    q, k, v = _qkv(4800, rows, c0)
+    q, k, v = (q * np.float32(sq)).astype(np.float32), (k * np.float32(sk)).astype(np.float32), v * np.float32(sv)
+    v[::3] = 0.0
+    k[1::3] = 0.0
+    st, want = O.chunk_prefill_attention(q, k, v, NH, D, c0)
+    assert st == 0
+    _close(_run(ctx, q, k, v, c0), want)
