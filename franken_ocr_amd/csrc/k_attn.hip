@@ -112,11 +112,13 @@ __device__ __forceinline__ uint3 split2(float a, float b) {
     return make_uint3(w1, w2, pk_bf16(sub_lo(ar, w2), sub_hi(br, w2)));
 }
 
-// chk turns NaN (and stays so) where a first term is infinite or NaN: values
-// that have no split.
-__device__ __forceinline__ float chk_terms(float chk, uint32_t w1) {
-    return __builtin_amdgcn_fdot2_f32_bf16(__builtin_bit_cast(v2bf, w1), __builtin_bit_cast(v2bf, 0u), chk, false);
+// chk turns NaN or infinite (and stays so) where a first term is infinite or
+// NaN: values that have no split. times (two equal bf16) lowers the limit: with
+// 2^23 chk overflows from first terms of 2^104, or of 2^100 where they add up.
+__device__ __forceinline__ float chk_terms(float chk, uint32_t w1, uint32_t times) {
+    return __builtin_amdgcn_fdot2_f32_bf16(__builtin_bit_cast(v2bf, w1), __builtin_bit_cast(v2bf, times), chk, false);
 }
+__device__ __forceinline__ bool not_finite(float x) { return !(fabsf(x) < INFINITY); }
 
 // Below kMinSplit the third term runs out of bf16's range (its last bit is at
 // 2^-133; the least term of 2^-100 is at 2^-123, still a normal number), so
@@ -133,9 +135,9 @@ __device__ __forceinline__ bool too_low(float x) { return x != 0.0f && fabsf(x) 
 
 struct Split8 {
     v4u w[3];  // terms 1, 2, 3 of eight values
-    __device__ __forceinline__ void pair(int i, float a, float b, float& chk) {
+    __device__ __forceinline__ void pair(int i, float a, float b, float& chk, uint32_t times = 0u) {
         const uint3 t = split2(a, b);
-        chk = chk_terms(chk, t.x);
+        chk = chk_terms(chk, t.x, times);
         w[0][i] = t.x;
         w[1][i] = t.y;
         w[2][i] = t.z;
@@ -173,9 +175,18 @@ __device__ __forceinline__ float softmax_max(v16f& sm, const AttnArgs& a, int kb
     return m_use;
 }
 
+// Scores further from zero than this (base 2, as m_run) are left to the f32
+// products: the fast path's exponent, one fma of the unrounded product, is off
+// the rounded maximum by half an ulp of it, 2^-5 here, which all of a row's
+// probabilities share and the denominator takes out again. From 2^31 on it
+// would be past the exponents' range.
+constexpr float kFarScore = 0x1p20f;
+constexpr uint32_t kVLimit = 0x4b004b00u;  // 2^23 twice: V from 2^104, where a probability above 1 could overflow
+
 // A wave's whole key range on f32 MFMAs from memory, for blocks whose values
-// have no split: infinities and NaN come out as the f32 products give them.
-// The results have the fast path's layout.
+// have no split and for rows whose scores are far from zero: infinities and
+// NaN come out as the f32 products give them, and a range's largest score has
+// the probability 1 exactly. The results have the fast path's layout.
 __device__ __forceinline__ void attend_f32(const AttnArgs& a, int h, int ks, int ke, int t, int wrow0, int qrow,
                                            int lane, v16f (&oacc)[4], float& m_run, float& l_run) {
     const int hf = lane >> 5, j = lane & 31;
@@ -189,23 +200,31 @@ __device__ __forceinline__ void attend_f32(const AttnArgs& a, int h, int ks, int
     if (wrow0 >= a.cs) return;
     for (int kb = ks; kb < min(ke, a.c0 + wrow0 + 32); kb += kKT) {
         const float* kp = kh + static_cast<size_t>(min(kb + j, a.c1 - 1)) * a.ldk;
-        v16f sm = v16f(0.0f);
-#pragma unroll 4
-        for (int s = 0; s < kD; s += 2) sm = __builtin_amdgcn_mfma_f32_32x32x2f32(kp[s], qp[s], sm, 0, 0, 0);
+        // (the dot in four chains, the tile's outputs from zero: a value goes
+        // through no more roundings than in the other forms)
+        v16f sc[4] = {v16f(0.0f), v16f(0.0f), v16f(0.0f), v16f(0.0f)};
+#pragma unroll 2
+        for (int s = 0; s < kD / 4; s += 2)
+#pragma unroll
+            for (int c = 0; c < 4; ++c)
+                sc[c] = __builtin_amdgcn_mfma_f32_32x32x2f32(kp[32 * c + s], qp[32 * c + s], sc[c], 0, 0, 0);
+        v16f sm = (sc[0] + sc[1]) + (sc[2] + sc[3]);
         float corr;
         const float m_use = softmax_max(sm, a, kb, ke, t, wrow0, hf, m_run, corr);
-        l_run *= corr;
-#pragma unroll
-        for (int d = 0; d < 4; ++d) oacc[d] = oacc[d] * corr;
+        float tsum = 0.0f;
+        v16f o[4] = {v16f(0.0f), v16f(0.0f), v16f(0.0f), v16f(0.0f)};
 #pragma unroll
         for (int r = 0; r < 16; ++r) {
-            const float p = __builtin_amdgcn_exp2f(fmaf(sm[r], a.scale, -m_use));
-            l_run += p;
+            const float p = __builtin_amdgcn_exp2f(sm[r] * a.scale - m_use);
+            tsum += p;
             const float* vr = vh + static_cast<size_t>(min(kb + 8 * (r >> 2) + 4 * hf + (r & 3), a.c1 - 1)) * a.ldv;
 #pragma unroll
             for (int d = 0; d < 4; ++d)
-                oacc[d] = __builtin_amdgcn_mfma_f32_32x32x2f32(vr[32 * d], p, oacc[d], 0, 0, 0);
+                o[d] = __builtin_amdgcn_mfma_f32_32x32x2f32(vr[32 * d], p, o[d], 0, 0, 0);
         }
+        l_run = l_run * corr + tsum;
+#pragma unroll
+        for (int d = 0; d < 4; ++d) oacc[d] = oacc[d] * corr + o[d];
     }
 }
 
@@ -313,6 +332,7 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(kBlocksPerC
     };
     auto store_v = [&]() {
         float chk = 0.0f, low = INFINITY;
+        const uint32_t limit = opaque(kVLimit);
 #pragma unroll
         for (int i = 0; i < 8; ++i) low = low_abs(low, pv[i].x, pv[i].y);
         if (low < kMinSplit) {
@@ -325,13 +345,13 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(kBlocksPerC
             Split8 s;
 #pragma unroll
             for (int i = 0; i < 4; ++i)
-                s.pair(i, pv[2 * i][e], pv[2 * i + 1][e], chk);
+                s.pair(i, pv[2 * i][e], pv[2 * i + 1][e], chk, limit);
             const int d = (2 * lane + e) & 31;
             const int slot = ((wave >> 1) * 4 + (lane >> 4)) * kVFrag + (wave & 1) * 32 + (d ^ ((d >> 3) & 1));
 #pragma unroll
             for (int m = 0; m < 3; ++m) lv[m * kVTerm + slot] = s.w[m];
         }
-        if (chk != chk) bad[1] = 1;
+        if (not_finite(chk)) bad[1] = 1;
     };
 
     load_k(ks);
@@ -377,7 +397,8 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(kBlocksPerC
     store_k();
     load_v(ks);
 
-    bool no_split = false;  // block-uniform
+    bool no_split = false;    // block-uniform
+    unsigned long long far = 0;  // lanes whose scores were far from zero
     for (int kb = ks; kb < ke; kb += kKT) {
         const bool live = wrow0 < a.cs && kb <= a.c0 + wrow0 + 31;  // wave-uniform: some row sees some key
         __syncthreads();  // K(kb) staged; every wave is done with V of the tile before
@@ -414,6 +435,7 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(kBlocksPerC
             }
             sm = sm + sl;
             const float m_use = softmax_max(sm, a, kb, ke, t, wrow0, hf, m_run, corr);
+            far |= __builtin_amdgcn_ballot_w64(fabsf(m_use) > kFarScore);
             float tsum = 0.0f;
 #pragma unroll
             for (int i = 0; i < 8; ++i) {
@@ -462,7 +484,11 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(kBlocksPerC
             }
         }
     }
-    if (no_split) attend_f32(a, h, ks, ke, t, wrow0, qrow, lane, oacc, m_run, l_run);
+    // a score that overflowed (a sum of first terms can where the f32 dot does
+    // not, and the two sums with opposite signs) shows as a denominator that is
+    // not finite, or as a row with keys and no maximum
+    far |= __builtin_amdgcn_ballot_w64(not_finite(l_run) || (m_run == -INFINITY && ks <= t));
+    if (no_split || far) attend_f32(a, h, ks, ke, t, wrow0, qrow, lane, oacc, m_run, l_run);
     float other;
     l_run = perm32(l_run, other) + other;
     __syncthreads();  // the staging becomes the waves' output rows

@@ -134,3 +134,45 @@ def test_values_too_small_for_three_bf16_terms(ctx, rows, c0, sq, sk, sv):
     st, want = O.chunk_prefill_attention(q, k, v, NH, D, c0)
     assert st == 0
     _close(_run(ctx, q, k, v, c0), want)
+
+
+def _f32_rows(q, k, v, c0):
+    """The attention in f32 scores: for scores so large that f32 decides which
+    key is the row's largest, the f64 softmax of the f32 scores."""
+    out = np.empty(q.shape, np.float64)
+    for h in range(NH):
+        cols = slice(h * D, (h + 1) * D)
+        for i in range(q.shape[0]):
+            s = (k[:c0 + i + 1, cols].astype(np.float64) @ q[i, cols].astype(np.float64)).astype(np.float32)
+            s = s.astype(np.float64) / np.sqrt(D)
+            p = np.exp(s - s.max())
+            out[i, cols] = p @ v[:c0 + i + 1, cols].astype(np.float64) / p.sum()
+    return out
+
+
+@pytest.mark.parametrize("rows,c0", [(40, 60), (260, 95)])
+@pytest.mark.parametrize("scale", [1e5, 1e12, 1e18])
+def test_scores_far_from_zero(ctx, rows, c0, scale):
+    """q and k of about that size: one key has all of a row's probability, and
+    the outputs are its value, whatever the scores' ulp (1e5: of 2^13, 1e12: of
+    2^59). A key is close enough to a row's largest to share it in none of them
+    (their gaps are some 1e-4 of the scores at the least)."""
+    q, k, v = _qkv(4900, rows, c0)
+    q, k = q * np.float32(scale), k * np.float32(scale)
+    _close(_run(ctx, q, k, v, c0), _f32_rows(q, k, v, c0))
+
+
+@pytest.mark.parametrize("rows,c0", [(40, 60), (260, 95), (300, 700)])
+def test_scores_that_overflow_downwards(ctx, rows, c0):
+    """Keys whose score is below f32's range have no probability; a row's other
+    keys are attended as ever (the last 20 columns of every 64 keys are such)."""
+    q, k, v = _qkv(5000, rows, c0)
+    low = np.arange(rows + c0) % 64 >= 44
+    q[:, 4::D] = 1e21
+    k[:, 4::D] = 0.0
+    less = k.copy()
+    less[low, 4::D] = -1e10  # as little probability, within range
+    st, want = O.chunk_prefill_attention(q, less, v, NH, D, c0)
+    assert st == 0 and np.isfinite(want).all()
+    k[low, 4::D] = -1e21 * synth.f32_uniform(synth.seed_of(5003), low.sum() * NH, 1.0, 1.02).reshape(-1, NH)
+    _close(_run(ctx, q, k, v, c0), want)
