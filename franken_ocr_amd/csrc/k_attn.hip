@@ -795,10 +795,10 @@ __device__ __forceinline__ float4 merge_row(const AttnArgs& a, int row, int h, i
     float4 acc = make_float4(0.0f, 0.0f, 0.0f, 0.0f);
     for (int s0 = 0; s0 < ns; s0 += 32) {
         const int n = min(ns - s0, 32);
-        float w = 0.0f;
+        float w = -1.0f;  // a range without a key of the row
         if (c < n) {
             const float2 ml = *reinterpret_cast<const float2*>(a.part_ml + (p0 + (s0 + c) * step) * 2);
-            w = ml.x == -INFINITY ? 0.0f : __builtin_amdgcn_exp2f(ml.x - M);
+            if (ml.x != -INFINITY) w = __builtin_amdgcn_exp2f(ml.x - M);
             den += ml.x == -INFINITY ? 0.0f : w * ml.y;
         }
         for (int s = 0; s < n; s += 4) {
@@ -806,19 +806,20 @@ __device__ __forceinline__ float4 merge_row(const AttnArgs& a, int row, int h, i
             float ws[4];
 #pragma unroll
             for (int i = 0; i < 4; ++i) {
-                const int si = min(s + i, n - 1);  // past the last: its output again, with weight 0
+                const int si = min(s + i, n - 1);  // past the last: its output again, not added
                 o[i] = *reinterpret_cast<const float4*>(a.part_o + (p0 + (s0 + si) * step) * kD + 4 * c);
                 ws[i] = __shfl(w, si, 32);
-                if (s + i >= n) ws[i] = 0.0f;
+                if (s + i >= n) ws[i] = -1.0f;
             }
 #pragma unroll
             for (int i = 0; i < 4; ++i) {
                 // (a range without a key of the row adds nothing, whatever the
-                // outputs of the other rows of its tile made of V)
-                acc.x += ws[i] != 0.0f ? ws[i] * o[i].x : 0.0f;
-                acc.y += ws[i] != 0.0f ? ws[i] * o[i].y : 0.0f;
-                acc.z += ws[i] != 0.0f ? ws[i] * o[i].z : 0.0f;
-                acc.w += ws[i] != 0.0f ? ws[i] * o[i].w : 0.0f;
+                // outputs of the other rows of its tile made of V; one whose
+                // weight is 0 adds 0 times its output, NaN where V is not finite)
+                acc.x += ws[i] < 0.0f ? 0.0f : ws[i] * o[i].x;
+                acc.y += ws[i] < 0.0f ? 0.0f : ws[i] * o[i].y;
+                acc.z += ws[i] < 0.0f ? 0.0f : ws[i] * o[i].z;
+                acc.w += ws[i] < 0.0f ? 0.0f : ws[i] * o[i].w;
             }
         }
     }

@@ -176,3 +176,18 @@ def test_scores_that_overflow_downwards(ctx, rows, c0):
     assert st == 0 and np.isfinite(want).all()
     k[low, 4::D] = -1e21 * synth.f32_uniform(synth.seed_of(5003), low.sum() * NH, 1.0, 1.02).reshape(-1, NH)
     _close(_run(ctx, q, k, v, c0), want)
+
+
+@pytest.mark.parametrize("bad", [np.inf, np.nan])
+@pytest.mark.parametrize("rows,c0", [(64, 440), (260, 95), (300, 700)])
+def test_a_value_that_is_not_finite_shows_at_probability_zero(ctx, rows, c0, bad):
+    """A key so far below the rows' largest score that its probability is 0 in
+    f32: 0 * inf and 0 * NaN are NaN, also where its whole key range (key 0's:
+    every key but the last 40) is that far below."""
+    q, k, v = _qkv(5100, rows, c0)
+    q[:, 4::D], k[:, 4::D] = 40.0, 0.0
+    k[c0 - 40:c0, 4::D] = 60.0  # + 212 in these keys' scores
+    v[0, 5] = bad
+    got = _run(ctx, q, k, v, c0)
+    assert np.isnan(got[:, 5]).all()
+    assert np.isfinite(np.delete(got, 5, 1)).all()
