@@ -248,12 +248,12 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(kBlocksPerC
     const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
     const int lane = threadIdx.x & 63;
     const int hf = lane >> 5, j = lane & 31;
-    const int h = blockIdx.x;
-    // the block's row tile and key range: blockIdx.y counts the ranges that
-    // have keys, the last row tile's first (they are the most and the
-    // longest); heads vary fastest, so the XCDs (block id % 8) share every
+    // the block's head, row tile and key range: blockIdx.x / heads counts the
+    // ranges that have keys, the last row tile's first (they are the most and
+    // the longest); heads vary fastest, so the XCDs (block id % 8) share every
     // row tile's work
-    int tile = (a.cs - 1) / kRT, split = blockIdx.y;
+    const int h = static_cast<int>(blockIdx.x % static_cast<unsigned>(a.heads));
+    int tile = (a.cs - 1) / kRT, split = static_cast<int>(blockIdx.x / static_cast<unsigned>(a.heads));
     for (; tile > 0; --tile) {
         const int ns = attn_ranges(a, tile * kRT);
         if (split < ns) break;
@@ -960,6 +960,13 @@ size_t attn_partials_bytes(int cs, int heads, int nsplit) {
 // Rows and keys for which attn_prefill_small_kernel is taken (measured beside it)
 static bool attn_small(int cs, int c1) { return cs <= 192 && c1 <= 512 && cs * c1 <= 65536; }
 
+// The partials a call may ask scratch for. By time alone the range length grows
+// slower than the call: 32768 rows asked for 3.2 GB, 131072 for 25 GB. Past the
+// limit ranges get longer, down to one a row tile, which has no partials, and
+// cost nothing that shows: 8192 rows (511 MB before) 1.09 to 1.11 ms, 16384
+// (1.1 GB) 3.94 to 3.84, 65536 (9.2 GB) 62.1 to 55.0.
+constexpr size_t kMaxPartials = size_t(512) << 20;
+
 int attn_pick_splits(int cs, int c1, int heads, int cu_count, int* split_len) {
     if (attn_small(cs, c1)) {
         // the shortest ranges whose blocks are resident at once
@@ -990,6 +997,7 @@ int attn_pick_splits(int cs, int c1, int heads, int cu_count, int* split_len) {
     double best = 0.0;
     int per = tiles;  // tiles per range
     for (int p = 1; p <= tiles; p += 1 + p / 16) {
+        if (p < tiles && attn_partials_bytes(cs, heads, (tiles + p - 1) / p) > kMaxPartials) continue;
         double blocks = 0.0, part_rows = 0.0;
         for (int r = 0; r < cs; r += kRT) {
             const int n = (min(c1, c0 + r + kRT) + kKT - 1) / kKT, ranges = (n + p - 1) / p;
@@ -1026,7 +1034,7 @@ hipError_t launch_attn_prefill(hipStream_t s, const AttnGeom& gm, const float* q
     } else {
         int ranges = 0;
         for (int r = 0; r < cs; r += kRT) ranges += (min(c1, c0 + r + kRT) + split_len - 1) / split_len;
-        FOCR_LAUNCH(attn_prefill_kernel, dim3(heads, ranges), dim3(256), 0, s, a);
+        FOCR_LAUNCH(attn_prefill_kernel, dim3(static_cast<unsigned>(heads) * ranges), dim3(256), 0, s, a);
     }
     hipError_t e = hipGetLastError();
     if (qo) qo->done = false;

@@ -8,6 +8,8 @@ these tests runs on both, 260 rows after 95 and 300 after 700 being past it."""
 
 from __future__ import annotations
 
+import ctypes
+
 import numpy as np
 import pytest
 
@@ -191,3 +193,28 @@ def test_a_value_that_is_not_finite_shows_at_probability_zero(ctx, rows, c0, bad
     got = _run(ctx, q, k, v, c0)
     assert np.isnan(got[:, 5]).all()
     assert np.isfinite(np.delete(got, 5, 1)).all()
+
+
+def test_a_long_call_keeps_its_partials_within_bounds(ctx):
+    """32768 rows over 32768 keys: the key ranges' partials stay within 512 MiB
+    of scratch (ranges as short as the time alone asks for would take 3.2 GB),
+    and the rows are right."""
+    from franken_ocr_amd.engine import chunk_prefill_attention
+
+    rows = 32768
+    path = next(ln.split()[-1] for ln in open("/proc/self/maps") if "libamdhip64" in ln)
+    hip, free, total = ctypes.CDLL(path), ctypes.c_size_t(), ctypes.c_size_t()
+    x = np.tile(synth.f32_normal(synth.seed_of(5200), 512 * DIM).reshape(512, DIM), (rows // 512, 1))
+    dx, out = ctx.to_device(x), ctx.empty((rows, DIM), np.float32)
+    assert hip.hipMemGetInfo(ctypes.byref(free), ctypes.byref(total)) == 0
+    before = free.value
+    chunk_prefill_attention(dx, dx, dx, NH, D, 0, out)
+    got = out.numpy()
+    assert hip.hipMemGetInfo(ctypes.byref(free), ctypes.byref(total)) == 0
+    assert before - free.value <= (512 << 20) + (64 << 20), before - free.value
+    for row in (0, 4097, 20000, rows - 1):
+        keys = x[:row + 1].reshape(-1, NH, D)
+        s = np.einsum("khd,hd->hk", keys, x[row].reshape(NH, D), dtype=np.float64) / np.sqrt(D)
+        p = np.exp(s - s.max(axis=1, keepdims=True))
+        p /= p.sum(axis=1, keepdims=True)
+        _close(got[row], np.einsum("hk,khd->hd", p, keys, dtype=np.float64).reshape(-1))
