@@ -1076,55 +1076,81 @@ extern "C" {
 // the split-K GEMV in 16-row groups on the upload layout where it is the
 // faster, else up to 255 rows 64-row tiles on the fragment-order weight copy;
 // either gives way to the tiled-order GEMMs where i8_gemm_tiled_preferred, and
-// those run everything else. Rows that could go either way stay off the tiled
-// order in a call captured into a graph before the handle has its tiled
-// weights, which cannot be allocated then.
+// those run everything else.
+//
+// The copies are made by the first call that takes them, which a call captured
+// into a graph cannot do. Such a call takes what the handle has: rows that
+// could go either way stay off the tiled order until it is there, and rows
+// that would take the fragment order take the tiled one where only that is (a
+// call of more rows made it; the tiled GEMMs run any number). A GEMV call whose
+// tiled copy finds no memory runs the GEMV, which needs none.
 enum class LinearRoute { kTiled, kGemv, kFragments };
+
+static bool stream_captures(focr_hip_ctx* ctx) {
+    hipStreamCaptureStatus cap = hipStreamCaptureStatusNone;
+    return hipStreamIsCapturing(ctx->stream, &cap) != hipSuccess || cap != hipStreamCaptureStatusNone;
+}
+
+// The weights in the tiled order.
+static int32_t ensure_linear_tiled(focr_hip_ctx* ctx, const focr_hip_qint8* w) {
+    if (w->w_tiled) return FOCR_HIP_OK;
+    const size_t bytes = i8_gemm256_b_bytes((int)w->n, (int)w->k);
+    int8_t* p = nullptr;
+    if (hipMalloc(&p, bytes) != hipSuccess) {
+        (void)hipGetLastError();  // not the next launch's
+        return fail(FOCR_HIP_E_OOM, fmt("linear_int8_dynamic: tiled weight copy of %zu bytes", bytes));
+    }
+    hipError_t e = launch_i8_gemm256_retile_b(ctx->stream, w->w, (int)w->n, (int)w->k, p);
+    if (e != hipSuccess) {
+        hipFree(p);
+        return hip_fail(e, "retile launch");
+    }
+    w->w_tiled = p;
+    return FOCR_HIP_OK;
+}
+
 static LinearRoute linear_i8_route(focr_hip_ctx* ctx, const focr_hip_qint8* w, size_t m, const float* bias) {
     const int n = (int)w->n, k = (int)w->k;
     const bool gemv = !bias && gemv_rows_preferred(n, k, (int)m, false);
     const LinearRoute other = gemv ? LinearRoute::kGemv : LinearRoute::kFragments;
     if (!i8_gemm_tiled_supported((int)m, n, k)) return other;
     if (!gemv && m >= 256) return LinearRoute::kTiled;
-    if (!i8_gemm_tiled_preferred((int)m, n, k, ctx->cu_count)) return other;
+    if (!i8_gemm_tiled_preferred((int)m, n, k, ctx->cu_count))
+        return !gemv && !w->w_mfma && w->w_tiled && stream_captures(ctx) ? LinearRoute::kTiled : other;
     if (w->w_tiled) return LinearRoute::kTiled;
-    hipStreamCaptureStatus cap = hipStreamCaptureStatusNone;
-    const hipError_t e = hipStreamIsCapturing(ctx->stream, &cap);
-    return e == hipSuccess && cap == hipStreamCaptureStatusNone ? LinearRoute::kTiled : other;
+    return !stream_captures(ctx) && ensure_linear_tiled(ctx, w) == FOCR_HIP_OK ? LinearRoute::kTiled : other;
 }
 
-// norm_w (nullable): x is first RMS-normalised with that weight and eps, in
-// the quantize launch; only on the tiled path (the caller checks
-// linear_i8_norm_fusable)
+// Whether the input norm can run inside the quantize launch: on the tiled path.
 static bool linear_i8_norm_fusable(focr_hip_ctx* ctx, const focr_hip_qint8* w, size_t m) {
     return w && linear_i8_route(ctx, w, m, nullptr) == LinearRoute::kTiled && w->k <= 4096;
 }
 
-// The activation layout linear_int8_dynamic quantizes x into (row-major, or
-// the tiled order) and its bytes, in the kScrXq slot.
-static bool linear_i8_act_tiled(focr_hip_ctx* ctx, const focr_hip_qint8* w, size_t m, const float* bias) {
-    return linear_i8_route(ctx, w, m, bias) == LinearRoute::kTiled;
-}
-static size_t linear_i8_act_bytes(focr_hip_ctx* ctx, const focr_hip_qint8* w, size_t m, const float* bias) {
-    return linear_i8_act_tiled(ctx, w, m, bias) ? i8_gemm256_a_bytes((int)m, (int)w->k) : m * w->k;
+// Bytes of m rows as that route quantizes them (row-major, or the tiled
+// order), in the kScrXq slot.
+static size_t linear_i8_act_bytes(LinearRoute route, const focr_hip_qint8* w, size_t m) {
+    return route == LinearRoute::kTiled ? i8_gemm256_a_bytes((int)m, (int)w->k) : m * w->k;
 }
 
-// prequant: the rows are already quantized by the dynamic rule in the
-// kScrXq / kScrXs slots, in linear_i8_act_tiled's layout (x unused)
+// norm_w (nullable): x is first RMS-normalised with that weight and eps, in
+// the quantize launch; only on the tiled path (the caller checks
+// linear_i8_norm_fusable).
+// prequant (nullable): the rows are already quantized by the dynamic rule in
+// the kScrXq / kScrXs slots, for that route (x unused).
 static int32_t linear_i8_dynamic_impl(focr_hip_ctx* ctx, const focr_hip_qint8* w, const float* x, size_t m,
                                    const float* bias, float* y, const float* norm_w = nullptr, float eps = 0.0f,
-                                   bool prequant = false) {
+                                   const LinearRoute* prequant = nullptr) {
     if (!w) return fail(FOCR_HIP_E_BAD_HANDLE, "linear_int8_dynamic: null weight handle");
     if ((!x && !prequant) || !y) return fail(FOCR_HIP_E_ARG, "linear_int8_dynamic: null device pointer");
     if (m < 1 || m > (1u << 20)) return fail(FOCR_HIP_E_SHAPE, fmt("linear_int8_dynamic: m %zu outside 1..=1048576", m));
     if (!i8_mfma_supported(static_cast<int>(w->k)))
         return fail(FOCR_HIP_E_SHAPE,
                     fmt("linear_int8_dynamic: k %zu is not a multiple of 64 (the matrix-core K stage)", w->k));
-    if (norm_w && !linear_i8_norm_fusable(ctx, w, m))
+    const LinearRoute route = prequant ? *prequant : linear_i8_route(ctx, w, m, bias);
+    if (norm_w && (route != LinearRoute::kTiled || w->k > 4096))
         return fail(FOCR_HIP_E_ARG, "linear_int8_dynamic: the fused norm needs the tiled path");
-    const LinearRoute route = linear_i8_route(ctx, w, m, bias);
     if (route == LinearRoute::kGemv) {
-        int8_t* xq = static_cast<int8_t*>(ctx->scratch_get(kScrXq, m * w->k));
+        int8_t* xq = static_cast<int8_t*>(ctx->scratch_get(kScrXq, linear_i8_act_bytes(route, w, m)));
         float* xs = static_cast<float*>(ctx->scratch_get(kScrXs, m * sizeof(float)));
         if (!xq || !xs) return FOCR_HIP_E_OOM;
         if (!prequant) {
@@ -1138,25 +1164,10 @@ static int32_t linear_i8_dynamic_impl(focr_hip_ctx* ctx, const focr_hip_qint8* w
         return FOCR_HIP_OK;
     }
     const bool big = route == LinearRoute::kTiled;
-    if (big) {
-        if (!w->w_tiled) {
-            const size_t bytes = i8_gemm256_b_bytes((int)w->n, (int)w->k);
-            int8_t* p = nullptr;
-            if (hipMalloc(&p, bytes) != hipSuccess)
-                return fail(FOCR_HIP_E_OOM, fmt("linear_int8_dynamic: tiled weight copy of %zu bytes", bytes));
-            hipError_t e = launch_i8_gemm256_retile_b(ctx->stream, w->w, (int)w->n, (int)w->k, p);
-            if (e != hipSuccess) {
-                hipFree(p);
-                return hip_fail(e, "retile launch");
-            }
-            w->w_tiled = p;
-        }
-    } else {
-        int32_t st = ensure_tiled(ctx, &w->w_mfma, w->w, 1, w->n, w->k, "linear_int8_dynamic");
-        if (st) return st;
-    }
-    int8_t* xq = static_cast<int8_t*>(
-        ctx->scratch_get(kScrXq, big ? i8_gemm256_a_bytes((int)m, (int)w->k) : m * w->k));
+    int32_t st = big ? ensure_linear_tiled(ctx, w)
+                     : ensure_tiled(ctx, &w->w_mfma, w->w, 1, w->n, w->k, "linear_int8_dynamic");
+    if (st) return st;
+    int8_t* xq = static_cast<int8_t*>(ctx->scratch_get(kScrXq, linear_i8_act_bytes(route, w, m)));
     float* xs = static_cast<float*>(ctx->scratch_get(kScrXs, m * sizeof(float)));
     if (!xq || !xs) return FOCR_HIP_E_OOM;
     if (!prequant) {
@@ -1904,14 +1915,15 @@ static int32_t decoder_layer_prefill_impl(focr_hip_ctx* ctx, const focr_hip_deco
     // the split merge writes the context rows quantized for o_proj, in the
     // layout and scratch o_proj's linear_int8_dynamic reads
     AttnQuantOut qo{};
-    qo.tiled = linear_i8_act_tiled(ctx, L->o_proj, cs, nullptr);
-    qo.xq = static_cast<int8_t*>(ctx->scratch_get(kScrXq, linear_i8_act_bytes(ctx, L->o_proj, cs, nullptr)));
+    const LinearRoute o_route = linear_i8_route(ctx, L->o_proj, cs, nullptr);
+    qo.tiled = o_route == LinearRoute::kTiled;
+    qo.xq = static_cast<int8_t*>(ctx->scratch_get(kScrXq, linear_i8_act_bytes(o_route, L->o_proj, cs)));
     qo.xs = static_cast<float*>(ctx->scratch_get(kScrXs, cs * sizeof(float)));
     if (!qo.xq || !qo.xs) return FOCR_HIP_E_OOM;
     if ((st = rswa_prefill_chunk_impl(ctx, cache, stream, q, nullptr, nullptr, cs, c0, cx, true, &qo))) return st;
     // 5. o_proj; 6. residual + post-attention RMSNorm
     if ((st = linear_i8_dynamic_impl(ctx, L->o_proj, qo.done ? nullptr : cx, cs, nullptr, attn, nullptr, 0.0f,
-                                     qo.done)))
+                                     qo.done ? &o_route : nullptr)))
         return st;
     {
         ProfScope ps(ctx, "layer_prefill_residual_norm");

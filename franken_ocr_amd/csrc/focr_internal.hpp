@@ -131,11 +131,10 @@ struct focr_hip_qint8 {
     float* scales = nullptr;
     size_t n = 0, k = 0;
     bool owned = false;
-    // the weights in the matrix-core fragment order (launch_retile_i8), built
-    // the first time the handle is used for prefill; always owned
+    // the weights in the matrix-core fragment order (launch_retile_i8) and in
+    // the tiled GEMMs' order (launch_i8_gemm256_retile_b), each built by the
+    // first linear_int8_dynamic whose rows take it (linear_i8_route); always owned
     mutable int8_t* w_mfma = nullptr;
-    // the weights in the large-row GEMM's tiled order (launch_i8_gemm256_retile_b),
-    // built the first time the handle multiplies 256 rows or more; always owned
     mutable int8_t* w_tiled = nullptr;
 };
 
@@ -582,9 +581,9 @@ hipError_t launch_retile_i8(hipStream_t s, const int8_t* src, int n_mats, int n,
 // on rows already quantized by the dynamic rule; w in fragment order.
 hipError_t launch_linear_i8(hipStream_t s, const int8_t* xq, const float* xs, int m, int k, const int8_t* w,
                             const float* ws, int n, const float* bias, float* y);
-// k_i8gemm.hip — the same product for large row counts: 256 x 128 block
-// tiles, both operands in a tiled order (the activations written so by the
-// quantizer, the weights retiled once). Needs m >= 256 and k a multiple of 64.
+// k_i8gemm.hip — the same product in 256 x 128 or 64 x 64 blocks, both operands
+// in a tiled order (the activations written so by the quantizer, in tiles of
+// 256 rows, the weights retiled once). Any m; k a multiple of 64.
 bool i8_gemm_tiled_supported(int m, int n, int k);
 bool i8_gemm_tiled_preferred(int m, int n, int k, int cu_count);  // where another kernel could run too
 size_t i8_gemm256_a_bytes(int m, int k);  // tiled activation buffer

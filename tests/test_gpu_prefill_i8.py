@@ -258,7 +258,6 @@ def test_linear_i8_captured_before_the_tiled_weights(ctx, m, k, n):
     from franken_ocr_amd.engine import QInt8, linear_i8_dynamic
 
     _say(f"captured linear m={m} k={k} n={n}")
-    hip, ct = _hip()
     x = synth.f32_normal(synth.seed_of(9900 + m), m * k).reshape(m, k)
     w = synth.int8_uniform(synth.seed_of(9901), n * k)
     ws = synth.f32_uniform(synth.seed_of(9902), n, 1e-3, 2e-2)
@@ -272,18 +271,50 @@ def test_linear_i8_captured_before_the_tiled_weights(ctx, m, k, n):
         zero = ctx.to_device(np.zeros(n, np.float32))
         linear_i8_dynamic(q, ctx.to_device(x[:5]), ctx.empty((5, n), np.float32), zero)
     dz = ctx.to_device(np.zeros((m, n), np.float32))
-    ctx.synchronize()
+    _replays(ctx, lambda: linear_i8_dynamic(q, dx, dz), dz, want, 2)  # relaxed
+
+
+def _replays(ctx, call, out, want, mode):
+    """`call` captured in that mode, replayed three times."""
+    hip, ct = _hip()
     stream, graph, ex = ct.c_void_p(ctx.stream()), ct.c_void_p(), ct.c_void_p()
-    assert hip.hipStreamBeginCapture(stream, 2) == 0  # relaxed
+    ctx.synchronize()
+    assert hip.hipStreamBeginCapture(stream, mode) == 0
     try:
-        linear_i8_dynamic(q, dx, dz)
+        call()
     finally:
         rc = hip.hipStreamEndCapture(stream, ct.byref(graph))
     assert rc == 0
     assert hip.hipGraphInstantiate(ct.byref(ex), graph, None, None, ct.c_size_t(0)) == 0
     for _ in range(3):
+        out.copy_from(np.full(out.shape, 3.0, np.float32))
         assert hip.hipGraphLaunch(ex, stream) == 0
         ctx.synchronize()
-        assert np.array_equal(dz.numpy(), want)
+        assert np.array_equal(out.numpy(), want)
     hip.hipGraphExecDestroy(ex)
     hip.hipGraphDestroy(graph)
+
+
+@pytest.mark.parametrize("warm,m,k,n", [(64, 5, 1280, 4096), (255, 17, 1280, 1280), (256, 5, 128, 33000)])
+def test_linear_i8_captured_with_the_tiled_weights_alone(ctx, warm, m, k, n):
+    """A handle whose only call so far took the tiled order: a captured call of
+    fewer rows, whose own order is the fragments', cannot make that copy and
+    runs the tiled GEMM (the last shape in its 256-row blocks, five of them
+    filled), with the oracle's bits."""
+    from franken_ocr_amd.engine import QInt8, linear_i8_dynamic
+
+    _say(f"captured linear m={m} after m={warm} k={k} n={n}")
+    x = synth.f32_normal(synth.seed_of(9910 + m), warm * k).reshape(warm, k)
+    w = synth.int8_uniform(synth.seed_of(9911), n * k)
+    ws = synth.f32_uniform(synth.seed_of(9912), n, 1e-3, 2e-2)
+    b = synth.f32_normal(synth.seed_of(9913), n)
+    q, db, dx = QInt8(w, ws, n, k, ctx), ctx.to_device(b), ctx.to_device(x)
+    warmed = ctx.empty((warm, n), np.float32)
+    linear_i8_dynamic(q, dx, warmed, db)
+    st, want, _, _ = O.linear_i8_dynamic(x, w, ws, n, b)
+    assert st == 0 and np.array_equal(warmed.numpy(), want)
+    dy = ctx.empty((m, n), np.float32)
+    few = dx.view_rows(0, m)
+    _replays(ctx, lambda: linear_i8_dynamic(q, few, dy, db), dy, want[:m], 0)  # global: no allocation at all
+    linear_i8_dynamic(q, few, dy, db)  # and not captured
+    assert np.array_equal(dy.numpy(), want[:m])
