@@ -10,6 +10,7 @@
 #include <cstring>
 #include <limits>
 #include <memory>
+#include <mutex>
 #include <new>
 #include <string>
 #include <vector>
@@ -1091,8 +1092,13 @@ static bool stream_captures(focr_hip_ctx* ctx) {
     return hipStreamIsCapturing(ctx->stream, &cap) != hipSuccess || cap != hipStreamCaptureStatusNone;
 }
 
-// The weights in the tiled order.
+// The weights in the tiled order. The handle may be in use by calls of other
+// contexts, on streams and threads of their own: one of them makes the copy,
+// and it is complete before the handle shows it. (Inside a capture the copy is
+// part of the graph.)
 static int32_t ensure_linear_tiled(focr_hip_ctx* ctx, const focr_hip_qint8* w) {
+    static std::mutex one;
+    const std::lock_guard<std::mutex> lock(one);
     if (w->w_tiled) return FOCR_HIP_OK;
     const size_t bytes = i8_gemm256_b_bytes((int)w->n, (int)w->k);
     int8_t* p = nullptr;
@@ -1101,6 +1107,7 @@ static int32_t ensure_linear_tiled(focr_hip_ctx* ctx, const focr_hip_qint8* w) {
         return fail(FOCR_HIP_E_OOM, fmt("linear_int8_dynamic: tiled weight copy of %zu bytes", bytes));
     }
     hipError_t e = launch_i8_gemm256_retile_b(ctx->stream, w->w, (int)w->n, (int)w->k, p);
+    if (e == hipSuccess && !stream_captures(ctx)) e = hipStreamSynchronize(ctx->stream);
     if (e != hipSuccess) {
         hipFree(p);
         return hip_fail(e, "retile launch");

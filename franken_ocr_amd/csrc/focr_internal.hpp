@@ -6,6 +6,7 @@
 #include <hip/hip_ext.h>
 #include <hip/hip_runtime.h>
 
+#include <atomic>
 #include <cstddef>
 #include <cstdint>
 #include <map>
@@ -133,9 +134,10 @@ struct focr_hip_qint8 {
     bool owned = false;
     // the weights in the matrix-core fragment order (launch_retile_i8) and in
     // the tiled GEMMs' order (launch_i8_gemm256_retile_b), each built by the
-    // first linear_int8_dynamic whose rows take it (linear_i8_route); always owned
+    // first linear_int8_dynamic whose rows take it (linear_i8_route); always
+    // owned. w_tiled is complete before it is set, as other contexts may read it.
     mutable int8_t* w_mfma = nullptr;
-    mutable int8_t* w_tiled = nullptr;
+    mutable std::atomic<int8_t*> w_tiled{nullptr};
 };
 
 struct focr_hip_moe_layer {

@@ -318,3 +318,53 @@ def test_linear_i8_captured_with_the_tiled_weights_alone(ctx, warm, m, k, n):
     _replays(ctx, lambda: linear_i8_dynamic(q, few, dy, db), dy, want[:m], 0)  # global: no allocation at all
     linear_i8_dynamic(q, few, dy, db)  # and not captured
     assert np.array_equal(dy.numpy(), want[:m])
+
+
+def test_linear_i8_first_calls_from_two_contexts(ctx):
+    """Two threads, each with a context of its own, make a fresh handle's first
+    calls at once: the tiled weight copy is made once and complete for both."""
+    import threading
+
+    from franken_ocr_amd import _abi
+    from franken_ocr_amd.device import Context
+    from franken_ocr_amd.engine import QInt8
+
+    m, k, n = 64, 1280, 4096
+    _say(f"first calls of two contexts m={m} k={k} n={n}")
+    x = synth.f32_normal(synth.seed_of(9920), m * k).reshape(m, k)
+    w = synth.int8_uniform(synth.seed_of(9921), n * k)
+    ws = synth.f32_uniform(synth.seed_of(9922), n, 1e-3, 2e-2)
+    st, want, _, _ = O.linear_i8_dynamic(x, w, ws, n)
+    assert st == 0
+    contexts = [Context(0), Context(0)]
+    ins = [c.empty((m, k), np.float32).copy_from(x) for c in contexts]
+    outs = [c.empty((m, n), np.float32) for c in contexts]
+    for _ in range(4):
+        q = QInt8(w, ws, n, k, ctx)
+        ctx.synchronize()
+        start, errors = threading.Barrier(2), []
+
+        def call(i):
+            try:
+                start.wait()
+                _abi.call("focr_hip_linear_i8_dynamic", contexts[i].handle, q.handle, ins[i].c_ptr, m, None,
+                          outs[i].c_ptr)
+                contexts[i].synchronize()
+            except Exception as e:  # shown below, in the test's own thread
+                errors.append(e)
+
+        threads = [threading.Thread(target=call, args=(i,)) for i in range(2)]
+        for t in threads:
+            t.start()
+        for t in threads:
+            t.join()
+        assert not errors, errors
+        for out in outs:
+            assert np.array_equal(out.numpy(), want)
+        for c in contexts:
+            c.synchronize()
+        q.free()
+    for a in (*ins, *outs):
+        a.free()
+    for c in contexts:
+        c.close()
