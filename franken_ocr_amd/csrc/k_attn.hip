@@ -4,22 +4,22 @@
 // A chunk's cs queries (global positions c0 .. c0 + cs - 1) attend keys
 // [0, t] of the f32 prefix, per head, softmax(q.k * 1/sqrt(128)) . v.
 //
-// Every f32 operand x is the exact sum of three bf16 values, x = x1 + x2 + x3
+// An f32 operand x is the exact sum of three bf16 values, x = x1 + x2 + x3
 // (x1 = bf16(x), x2 = bf16(x - x1), x3 = x - x1 - x2: 8 + 8 + 8 bits of
 // mantissa, each residual exact), and a product x.y is the six MFMAs
 // x1y1 + x1y2 + x2y1 + x2y2 + x1y3 + x3y1, exact products summed in f32. The
-// three terms left out are below 2^-25 of |x||y|, half an f32 rounding, and
-// one v_mfma_f32_32x32x16_bf16 rounds once per 16 terms where the f32 MFMA
-// rounds once per 4: measured against 64 bits the attention is as near as the
-// f32 MFMA form or nearer. Six bf16 MFMAs take 6/16 of the f32 MFMA's matrix
+// three terms left out are at most 2^-24 of |x||y|, an f32 product's unit
+// roundoff. Measured against 64 bits the attention is nearer than in f32 MFMAs
+// (1024 rows 1.4e-7, 2.4e-7), and six bf16 MFMAs take 6/16 of their matrix
 // time. Values that have no such split (infinities, NaN, |x| so large that
-// bf16(x) is infinite) are found while staging, and their tiles take f32
-// MFMAs from memory (below).
+// bf16(x) is infinite, nonzero |x| below 2^-100, whose last terms bf16 does
+// not reach) are found while staging, and scores far from zero afterwards;
+// their ranges take f32 MFMAs from memory (attend_f32).
 //
 // Block = 4 waves on one head and 128 query rows (32 per wave); the block
 // walks its key range in tiles of 32 keys. The tile's K and V are split by
-// the threads that load them and staged in LDS in MFMA fragment order (24 KB
-// each, two blocks per CU at 256 VGPRs): K while the block's P.V of the tile
+// the threads that load them and staged in LDS in MFMA fragment order (25 KB
+// each, with 28 KB of Q terms two blocks per CU, at 256 VGPRs): K while the block's P.V of the tile
 // before runs, V while its scores run, so each load has a phase of MFMAs to
 // land in and one buffer of each is enough. Per wave S^T = K . Q^T (A = 32
 // keys x 16 dims from LDS, B = 16 dims x 32 query rows from registers, the
@@ -38,7 +38,7 @@
 // writes its running max, denominator and unnormalised output, and a merge
 // kernel folds them (log-sum-exp). A row whose keys all lie in other ranges
 // contributes max -inf and nothing else. The ranges hold equal numbers of
-// tiles, sized so the blocks that have keys fill the GPU about once (the
+// tiles, as many as make the least estimated time (attn_pick_splits; the
 // causal chunk's row tiles need different numbers of tiles).
 #include "focr_internal.hpp"
 #include "k_common.hpp"
@@ -49,7 +49,8 @@ namespace {
 constexpr int kD = 128;          // head_dim
 constexpr int kKT = 32;          // keys per LDS tile
 constexpr int kRT = 128;         // query rows per block
-constexpr int kBlocksPerCu = 2;  // the kernel's residency (LDS 48 KB, 256 VGPRs)
+constexpr int kBlocksPerCu = 2;  // the kernel's residency (LDS 77 KB, 256 VGPRs)
+constexpr int kCuLds = 160 * 1024;
 constexpr float kLog2e = 1.4426950408889634f;
 typedef float v4f __attribute__((ext_vector_type(4)));
 typedef float v2f __attribute__((ext_vector_type(2)));
@@ -245,6 +246,7 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(kBlocksPerC
     v4u* const lv = lk + 3 * kKTerm;
     // before and after the key loop: 32 rows of f32 per wave, one row's slots padded by one
     static_assert(4 * 32 * kORow <= 3 * kKTerm + 3 * kVTerm + 4 * kQLds * 64, "the waves' rows fit the staging");
+    static_assert(kBlocksPerCu * (sizeof(smem) + sizeof(bad)) <= kCuLds, "the blocks of a CU fit its LDS");
     const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
     const int lane = threadIdx.x & 63;
     const int hf = lane >> 5, j = lane & 31;
@@ -526,23 +528,18 @@ __device__ __forceinline__ float perm16_lo(float v, float& hi) {
     hi = __uint_as_float(r[1]);
     return __uint_as_float(r[0]);
 }
-__device__ __forceinline__ float perm32_lo(float v, float& hi) {
-    const auto r = __builtin_amdgcn_permlane32_swap(__float_as_uint(v), __float_as_uint(v), false, false);
-    hi = __uint_as_float(r[1]);
-    return __uint_as_float(r[0]);
-}
 __device__ __forceinline__ float wave16_max(float v) {
     float b;
     const float a = perm16_lo(v, b);
     v = fmaxf(a, b);
-    const float c = perm32_lo(v, b);
+    const float c = perm32(v, b);
     return fmaxf(c, b);
 }
 __device__ __forceinline__ float wave16_sum(float v) {
     float b;
     const float a = perm16_lo(v, b);
     v = a + b;
-    const float c = perm32_lo(v, b);
+    const float c = perm32(v, b);
     return c + b;
 }
 
@@ -551,7 +548,7 @@ __device__ __forceinline__ float wave16_sum(float v) {
 // its products, output, merge. The kernel above puts 128 query rows, their
 // splits and a pass through LDS for the output into that chain; this one has
 // 64 rows a block, 16 a wave, and exact f32 products on v_mfma_f32_16x16x4, so
-// its chain is shorter and its rate an eighth. Whole calls, this kernel and the
+// its chain is shorter and its matrix time 16/6. Whole calls, this kernel and the
 // one above, us: 16 rows 5.3, 8.1; 64 rows 10.1, 11.8; 128 rows 11.4, 18.6; 192
 // rows 13.3, 15.1; 64 rows after 448 keys 12.6, 16.3; 128 after 128 12.8, 15.3,
 // after 384 17.9, 18.7. Past that it loses: 256 rows 17.0, 16.4; 16 after 500
@@ -562,6 +559,7 @@ __device__ __forceinline__ float wave16_sum(float v) {
 // leave each lane 32 consecutive dims of its row. Ranges and partials are those
 // of the kernel above, so the merge is shared.
 constexpr int kSmRT = 64;                  // query rows per block
+constexpr int kSmKeys = 512;               // keys of a call at most
 constexpr int kSmBlocksPerCu = 3;          // residency (LDS 34 KB, 143 VGPRs)
 constexpr int kLdsRow = kD + 4;            // padded LDS row (floats)
 constexpr int kSub = kKT / 16;             // 16-key MFMA subtiles per tile
@@ -577,15 +575,15 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(kSmBlocksPe
     const int g = lane >> 4, j = lane & 15;
     const int h = blockIdx.y;
     const int split = blockIdx.z;
-    const int row0 = blockIdx.x * 64;            // block's first chunk row
-    const int wrow = row0 + wave * 16 + j;        // this lane's chunk row
+    const int row0 = blockIdx.x * kSmRT;         // block's first chunk row
+    const int wrow = row0 + wave * 16 + j;       // this lane's chunk row
     const int qrow = wrow < a.cs ? wrow : a.cs - 1;
     const int t = a.c0 + wrow;                    // its global position
-    // keys this block needs: [0, min(c1, c0 + row0 + 64)), this split's part
-    const int kmax = min(a.c1, a.c0 + row0 + 64);
+    // keys this block needs: [0, min(c1, c0 + row0 + kSmRT)), this split's part
+    const int kmax = min(a.c1, a.c0 + row0 + kSmRT);
     const int ks = split * a.split_len;
     const int ke = min(ks + a.split_len, kmax);
-    // a range past these 64 rows' last key; the merge goes by tiles of kRT
+    // a range past these rows' last key; the merge goes by tiles of kRT
     // rows, so it finds an empty range; block-uniform
     if (ks >= ke) {
         if (wrow < a.cs && g == 0 && ks < min(a.c1, a.c0 + (row0 / kRT + 1) * kRT))
@@ -638,10 +636,8 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(kSmBlocksPe
             *reinterpret_cast<v4f*>(lv + (r8 + 8 * p) * kLdsRow + 4 * c4) = pv[p];
         }
     };
-    if (ks < ke) {
-        load_tile(ks);
-        store_tile();
-    }
+    load_tile(ks);
+    store_tile();
     // every load so far (the Q fragment too) complete on every path into
     // the loop, so the loop's first MFMAs wait for none of the tile loads
     // issued inside it (vmcnt(0): the counter drains in issue order)
@@ -836,13 +832,13 @@ __global__ __launch_bounds__(256) void attn_merge_kernel(const AttnArgs a) {
         merge_row(a, row, h, c);
 }
 
-// The merge of attn_prefill_small_kernel's ranges (at most kSmRanges; a call
-// of more takes the kernel above): thread = one dim of one (row, head), every
-// range's (max, denominator) and output value requested at once, one round of
-// latency where the group form above has one per four ranges. 64 rows after 448
-// keys, whole call: 14.7 us with the form above, 12.5 with this; many rows pay
-// for the weights that every thread forms (1024 rows: 16 against 10 us).
-constexpr int kSmRanges = 16;
+// The merge of attn_prefill_small_kernel's ranges (at most kSmRanges): thread =
+// one dim of one (row, head), every range's (max, denominator) and output value
+// requested at once, one round of latency where the group form above has one
+// per four ranges. 64 rows after 448 keys, whole call: 14.7 us with the form
+// above, 12.5 with this; many rows pay for the weights that every thread forms
+// (1024 rows: 16 against 10 us).
+constexpr int kSmRanges = kSmKeys / kKT;
 
 __global__ __launch_bounds__(kD) void attn_merge_small_kernel(const AttnArgs a) {
     const int row = blockIdx.x, h = blockIdx.y, d = threadIdx.x;
@@ -958,7 +954,7 @@ size_t attn_partials_bytes(int cs, int heads, int nsplit) {
 }
 
 // Rows and keys for which attn_prefill_small_kernel is taken (measured beside it)
-static bool attn_small(int cs, int c1) { return cs <= 192 && c1 <= 512 && cs * c1 <= 65536; }
+static bool attn_small(int cs, int c1) { return cs <= 192 && c1 <= kSmKeys && cs * c1 <= 65536; }
 
 // The partials a call may ask scratch for. By time alone the range length grows
 // slower than the call: 32768 rows asked for 3.2 GB, 131072 for 25 GB. Past the
@@ -1048,7 +1044,7 @@ hipError_t launch_attn_prefill(hipStream_t s, const AttnGeom& gm, const float* q
         qo->done = true;
         return hipGetLastError();
     }
-    if (attn_small(cs, c1) && nsplit <= kSmRanges)
+    if (attn_small(cs, c1))
         FOCR_LAUNCH(attn_merge_small_kernel, dim3(cs, heads), dim3(kD), 0, s, a);
     else
         FOCR_LAUNCH(attn_merge_kernel, dim3((cs + 7) / 8, heads), dim3(256), 0, s, a);

@@ -218,3 +218,22 @@ def test_a_long_call_keeps_its_partials_within_bounds(ctx):
         p = np.exp(s - s.max(axis=1, keepdims=True))
         p /= p.sum(axis=1, keepdims=True)
         _close(got[row], np.einsum("hk,khd->hd", p, keys, dtype=np.float64).reshape(-1))
+
+
+@pytest.mark.parametrize("rows,c0", [(40, 60), (130, 382), (260, 95), (300, 700)])
+def test_rows_that_start_anywhere(ctx, rows, c0):
+    """q, k, v and the output four bytes past a 16-byte boundary: the same bits."""
+    from franken_ocr_amd.engine import chunk_prefill_attention
+
+    q, k, v = _qkv(5300, rows, c0)
+
+    def view(a):
+        buf = ctx.to_device(np.concatenate([np.zeros(1, np.float32), a.reshape(-1)]).reshape(-1, 1))
+        part = buf.view_rows(1, 1 + a.size)
+        part.shape = a.shape
+        assert part.ptr % 16 == 4
+        return part
+
+    out = view(np.zeros_like(q))
+    chunk_prefill_attention(view(q), view(k), view(v), NH, D, c0, out)
+    np.testing.assert_array_equal(out.numpy(), _run(ctx, q, k, v, c0))
