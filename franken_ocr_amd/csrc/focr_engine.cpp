@@ -1604,7 +1604,7 @@ static int32_t decoder_layer_step_impl(focr_hip_ctx* ctx, const focr_hip_decoder
     const size_t I = L->gate ? L->gate->n : 0;
     // one scratch slot carved into the step's intermediates
     const size_t fl = B * (3 * D + D + D + H + H + H) + (L->gate ? 3 * B * I : 0);
-    char* base = static_cast<char*>(ctx->scratch_get(kScrLayer, fl * 4 + B * H + B * I + 16 * 256));
+    char* base = static_cast<char*>(ctx->scratch_get(kScrLayer, fl * 4 + B * std::max(H, D) + B * I + 16 * 256));
     if (!base) return FOCR_HIP_E_OOM;
     auto take = [&](size_t bytes) {
         char* r = base;
@@ -1617,7 +1617,7 @@ static int32_t decoder_layer_step_impl(focr_hip_ctx* ctx, const focr_hip_decoder
     float* attn = reinterpret_cast<float*>(take(B * H * 4));
     float* h = reinterpret_cast<float*>(take(B * H * 4));
     float* nrm = reinterpret_cast<float*>(take(B * H * 4));
-    int8_t* xq = reinterpret_cast<int8_t*>(take(B * (H > D ? H : D)));
+    int8_t* xq = reinterpret_cast<int8_t*>(take(B * std::max(H, D)));
     float* xs = reinterpret_cast<float*>(take(B * 4));
     hipStream_t s = ctx->stream;
     // 1. input RMSNorm + quantize_row_i8, 2. the fused qkv GEMV, 3. RoPE at

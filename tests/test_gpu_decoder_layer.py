@@ -144,6 +144,44 @@ def test_decoder_layer_takes_rows_that_start_anywhere(ctx, kind, B):
     assert_rel(outs[1], outs[0], 1e-3)
 
 
+def test_decoder_layer_narrower_than_its_heads(ctx):
+    """hidden 640 under 10 heads x 128: the quantized rows of the contexts are
+    wider than those of x, and the step's scratch holds them. The separate
+    dense kernels (x off a 16-byte boundary) against the fused ones, eight
+    streams, and each against its stream stepped alone."""
+    from franken_ocr_amd.engine import DecoderLayer, QInt8, RingCache
+
+    h, n, B = 640, 6848, 8
+    _say(f"dense layer of hidden {h}, {B} streams")
+
+    def weight(seed, rows, k):
+        return QInt8(synth.int8_uniform(synth.seed_of(seed), rows * k),
+                     synth.f32_uniform(synth.seed_of(seed + 1), rows, 1e-3, 2e-2), rows, k, ctx)
+
+    layer = DecoderLayer(h, synth.f32_uniform(synth.seed_of(15000), h, 0.5, 1.5),
+                         synth.f32_uniform(synth.seed_of(15001), h, 0.5, 1.5), weight(15002, 3 * D, h),
+                         weight(15004, h, D), dense=(weight(15006, n, h), weight(15008, n, h), weight(15010, h, n)),
+                         ctx=ctx)
+    x = synth.f32_normal(synth.seed_of(15012), B * h)
+    pos = np.array([G + s for s in range(B)], np.uint32)
+    outs = []
+    for skip in (0, 1):
+        cache, _, kv = _prefill(ctx, B, 15100)
+        buf = ctx.to_device(np.concatenate([np.full(skip, 7.0, np.float32), x]).reshape(-1, 1))
+        rows = buf.view_rows(skip, skip + B * h)
+        layer.step(cache, pos, rows)
+        outs.append(rows.numpy().reshape(B, h))
+        cache.free()
+    assert_rel(outs[1], outs[0], 1e-3)
+    for s in (0, B - 1):
+        one = RingCache(1, G, ctx=ctx)
+        one.record_prefill(0, ctx.to_device(kv[s][0]), ctx.to_device(kv[s][1]), G)
+        row = ctx.to_device(np.ascontiguousarray(x.reshape(B, h)[s:s + 1]))
+        layer.step(one, pos[s:s + 1], row)
+        assert np.array_equal(row.numpy()[0], outs[0][s])
+        one.free()
+
+
 @pytest.mark.parametrize("kind,B", [("moe", 40), ("dense", 12)])
 def test_decoder_layer_more_streams_than_one_pass(ctx, kind, B):
     """More streams than one pass takes (32; 8 with the 6848-wide dense MLP)
