@@ -624,7 +624,10 @@ def cpu_rswa(args, inputs):
 # chunked prefill attention (decoder.rs:1282-1340), f32 precision
 # ---------------------------------------------------------------------------
 
-MFMA_F32_PEAK_TFLOPS = 157.3  # dense fp32 MFMA, MI355X
+# f32 products as six bf16 ones each (three-term splits of both operands) on
+# the dense bf16 MFMAs, MI355X: the form of every call past 192 rows or 512 keys
+MFMA_SPLIT_F32_PEAK_TFLOPS = round(2500.0 / 6, 1)
+MFMA_F64_PEAK_TFLOPS = 78.6  # the route's logits: f64, matrix and vector alike
 
 
 def attn_flops(seq: int, heads: int = 10, head_dim: int = 128) -> float:
@@ -666,7 +669,8 @@ def bench_prefill_attn(args, ctx):
         "config": {"workload": "prefill_attn", "seq": seq, "chunk": chunk, "heads": NH, "head_dim": D,
                    "chunks": len(bounds)},
         "roofline": {"bound": "mfma", "kernel": "attn_prefill", "achieved": round(achieved, 2),
-                     "peak": MFMA_F32_PEAK_TFLOPS, "unit": "TFLOP/s", "frac": round(achieved / MFMA_F32_PEAK_TFLOPS, 4),
+                     "peak": MFMA_SPLIT_F32_PEAK_TFLOPS, "unit": "TFLOP/s",
+                     "frac": round(achieved / MFMA_SPLIT_F32_PEAK_TFLOPS, 4),
                      "traffic": traffic_for("attn_prefill", f"prefill_attn_{seq}"), "algorithmic_flops_per_step": flops,
                      "avg_launch_us": round(a_us, 3), "launches_per_step": len(bounds), **launch_stats(prof, "attn_prefill")},
         "kernel_avg_us": kernels,
@@ -1234,23 +1238,23 @@ def bench_prefill_layer(args, ctx):
     gpu_out = x.numpy()
     counts = np.bincount(idx.numpy().ravel(), minlength=E)
     # algorithmic work per step: int8 products (2 ops per multiply-add) and
-    # the attention's f32 flops
+    # the attention's f32 and the route's f64 flops
     ops = {"linear_i8": 2.0 * seq * (3 * D * H + H * D),
            "i8_gate_up": 2.0 * seq * K * 2 * I * H, "i8_down": 2.0 * seq * K * H * I,
            "i8_shared": 2.0 * seq * 3 * SI * H}
     flops = {"attn_prefill": attn_flops(seq), "moe_route": 2.0 * seq * E * H}
     peak = {k: MFMA_INT8_PEAK_TOPS for k in ops}
-    peak.update({k: MFMA_F32_PEAK_TFLOPS for k in flops})
+    peak.update({"attn_prefill": MFMA_SPLIT_F32_PEAK_TFLOPS, "moe_route": MFMA_F64_PEAK_TFLOPS})
     work = {**ops, **flops}
     n_stat = max(args.steps, STAT_STEPS)  # steps of timed()'s per-kernel pass
     per_step = {k: (prof[k]["ms"] / n_stat if k in prof else float("nan")) for k in work}
     ideal_ms = sum(work[k] / (peak[k] * 1e12) * 1e3 for k in work)
     int8_ops = sum(ops.values())
     util = {
-        "int8_ops_per_step": int8_ops, "f32_flops_per_step": sum(flops.values()),
+        "int8_ops_per_step": int8_ops, "float_flops_per_step": sum(flops.values()),
         "ideal_ms_at_peak": round(ideal_ms, 5),
         # the fraction of the step a machine at MI355X's dense peaks would need
-        # for the same products (int8 at 5.0 POP/s, f32 at 157.3 TFLOP/s)
+        # for the same products (int8 at 5.0 POP/s, the others at their units')
         "frac_of_step": round(ideal_ms / ms, 4),
         "int8_tops_over_step": round(int8_ops / (ms * 1e-3) / 1e12, 2),
         "per_kernel": {k: {"ms_per_step": round(per_step[k], 5),
@@ -1501,11 +1505,12 @@ def bench_prefill(args, ctx):
     ms = el / args.steps * 1e3
     nb = len(prefill_chunk_bounds(seq, chunk or seq))
     # algorithmic work per step: int8 products (2 ops per multiply-add) and
-    # the attention's f32 flops
+    # the attention's f32 and the routes' f64 flops
     int8_ops = 2.0 * seq * (NL * (3 * D * H + H * D) + (NL - 1) * (K * 3 * I * H + 3 * SI * H) + 3 * ID * H) + \
         2.0 * V * H
-    f32_flops = NL * attn_flops(seq) + (NL - 1) * 2.0 * seq * E * H
-    ideal_ms = (int8_ops / (MFMA_INT8_PEAK_TOPS * 1e12) + f32_flops / (MFMA_F32_PEAK_TFLOPS * 1e12)) * 1e3
+    f32_flops, f64_flops = NL * attn_flops(seq), (NL - 1) * 2.0 * seq * E * H
+    ideal_ms = (int8_ops / (MFMA_INT8_PEAK_TOPS * 1e12) + f32_flops / (MFMA_SPLIT_F32_PEAK_TFLOPS * 1e12) +
+                f64_flops / (MFMA_F64_PEAK_TFLOPS * 1e12)) * 1e3
     weights = NL * (3 * D * H + H * D) + (NL - 1) * (E * 3 * I * H + 3 * SI * H) + 3 * ID * H + V * H
     log(f"per-kernel avg us {kernels}")
     return {
@@ -1518,7 +1523,7 @@ def bench_prefill(args, ctx):
                      "peak": MFMA_INT8_PEAK_TOPS, "unit": "TOP/s",
                      "frac": round(int8_ops / (ms * 1e-3) / 1e12 / MFMA_INT8_PEAK_TOPS, 4), "traffic": None,
                      "avg_step_us": round(ms * 1e3, 3)},
-        "mfma_utilisation": {"int8_ops_per_step": int8_ops, "f32_flops_per_step": f32_flops,
+        "mfma_utilisation": {"int8_ops_per_step": int8_ops, "float_flops_per_step": f32_flops + f64_flops,
                              "ideal_ms_at_peak": round(ideal_ms, 5), "frac_of_step": round(ideal_ms / ms, 4),
                              "weight_bytes_per_chunk": int(weights),
                              "weight_gbs_over_step": round(weights * nb / (ms * 1e-3) / 1e9, 1)},
@@ -1611,7 +1616,9 @@ _EXTRA_KEYS = ("layer_roofline", "mfma_utilisation", "layer_mfma", "kernel_avg_u
 def run_extras(ctx, base_args) -> dict:
     """Each secondary configuration timed like its own --workload run, then
     its CPU baseline on the host (base_args.extra_cpu_seconds each, unless
-    --no-cpu)."""
+    --no-cpu). The whole record of each goes to stderr; the result line holds
+    its figures in short, so that a reader who keeps the end of the output has
+    the line whole."""
     import gc
 
     out = {}
@@ -1641,7 +1648,10 @@ def run_extras(ctx, base_args) -> dict:
             ent["cpu_baseline"].update(host_cpu())
         else:
             ent["cpu_baseline"] = None
-        out[key] = ent
+        log(f"extra {key}: {json.dumps(ent)}")
+        out[key] = {**{k: ent[k] for k in ("value", "unit", "ms_per_step")}, "kernel": rl.get("kernel"),
+                    "achieved": rl.get("achieved"), "of": f"{rl.get('peak')} {rl.get('unit')}", "frac": rl.get("frac"),
+                    "traffic": rl.get("traffic"), "cpu": (ent["cpu_baseline"] or {}).get("value")}
         del res, cpu_inputs
         gc.collect()
     return out
