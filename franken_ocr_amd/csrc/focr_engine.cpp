@@ -13,6 +13,7 @@
 #include <mutex>
 #include <new>
 #include <string>
+#include <thread>
 #include <vector>
 
 #include "focr_internal.hpp"
@@ -211,6 +212,7 @@ int32_t focr_hip_qint8_free(focr_hip_qint8* w) {
     }
     hipFree(w->w_mfma);
     hipFree(w->w_tiled);
+    if (w->tiled_ready) hipEventDestroy(w->tiled_ready);
     delete w;
     return FOCR_HIP_OK;
 }
@@ -1092,26 +1094,45 @@ static bool stream_captures(focr_hip_ctx* ctx) {
     return hipStreamIsCapturing(ctx->stream, &cap) != hipSuccess || cap != hipStreamCaptureStatusNone;
 }
 
-// The weights in the tiled order. The handle may be in use by calls of other
-// contexts, on streams and threads of their own: one of them makes the copy,
-// and it is complete before the handle shows it. (Inside a capture the copy is
-// part of the graph.)
+// The weights in the tiled order, for a call of ctx. The handle may be in use
+// by calls of other contexts, on streams and threads of their own: one of them
+// makes the copy, and the others' first call waits until it is complete. (The
+// wait is the host's, once a handle, so that the maker's call waits for
+// nothing: synchronizing there made the first 1024-row prefill of twelve
+// layers 5.6 ms instead of 4.1.)
 static int32_t ensure_linear_tiled(focr_hip_ctx* ctx, const focr_hip_qint8* w) {
+    if (w->w_tiled && (ctx == w->tiled_by || w->tiled_done)) return FOCR_HIP_OK;
     static std::mutex one;
     const std::lock_guard<std::mutex> lock(one);
-    if (w->w_tiled) return FOCR_HIP_OK;
+    if (w->w_tiled) {
+        if (ctx == w->tiled_by || !w->tiled_ready) return FOCR_HIP_OK;
+        hipError_t e = hipSuccess;
+        while ((e = hipEventQuery(w->tiled_ready)) == hipErrorNotReady) std::this_thread::yield();
+        (void)hipGetLastError();  // not the next launch's
+        if (e != hipSuccess) return hip_fail(e, "tiled weight copy");
+        w->tiled_done = true;
+        return FOCR_HIP_OK;
+    }
     const size_t bytes = i8_gemm256_b_bytes((int)w->n, (int)w->k);
     int8_t* p = nullptr;
     if (hipMalloc(&p, bytes) != hipSuccess) {
-        (void)hipGetLastError();  // not the next launch's
+        (void)hipGetLastError();
         return fail(FOCR_HIP_E_OOM, fmt("linear_int8_dynamic: tiled weight copy of %zu bytes", bytes));
     }
+    hipEvent_t ready = nullptr;
     hipError_t e = launch_i8_gemm256_retile_b(ctx->stream, w->w, (int)w->n, (int)w->k, p);
-    if (e == hipSuccess && !stream_captures(ctx)) e = hipStreamSynchronize(ctx->stream);
+    if (e == hipSuccess && !stream_captures(ctx)) {
+        e = hipEventCreateWithFlags(&ready, hipEventDisableTiming);
+        if (e == hipSuccess) e = hipEventRecord(ready, ctx->stream);
+    }
     if (e != hipSuccess) {
+        hipStreamSynchronize(ctx->stream);
+        if (ready) hipEventDestroy(ready);
         hipFree(p);
         return hip_fail(e, "retile launch");
     }
+    w->tiled_by = ctx;
+    w->tiled_ready = ready;
     w->w_tiled = p;
     return FOCR_HIP_OK;
 }

@@ -135,9 +135,13 @@ struct focr_hip_qint8 {
     // the weights in the matrix-core fragment order (launch_retile_i8) and in
     // the tiled GEMMs' order (launch_i8_gemm256_retile_b), each built by the
     // first linear_int8_dynamic whose rows take it (linear_i8_route); always
-    // owned. w_tiled is complete before it is set, as other contexts may read it.
+    // owned. w_tiled is set once its launch is queued on tiled_by's stream;
+    // calls of other contexts wait for tiled_ready until tiled_done.
     mutable int8_t* w_mfma = nullptr;
     mutable std::atomic<int8_t*> w_tiled{nullptr};
+    mutable const focr_hip_ctx* tiled_by = nullptr;
+    mutable hipEvent_t tiled_ready = nullptr;  // null: made inside a capture, part of its graph
+    mutable std::atomic<bool> tiled_done{false};
 };
 
 struct focr_hip_moe_layer {
