@@ -182,7 +182,9 @@ int32_t focr_hip_igemm_s4s8_packed_dev(focr_hip_ctx* ctx, const int8_t* a,
 
 /* QInt8 weight handle (tensor.rs:149-179): w [n,k] i8 output-channel-major,
  * one f32 scale per output channel. _upload copies host arrays into HBM once;
- * _from_device wraps caller-owned device arrays (not freed by the handle). */
+ * _from_device wraps caller-owned device arrays (not freed by the handle),
+ * whose contents must stay as they are while the handle lives: prefill
+ * products read copies in other orders, made on the handle's first such call. */
 int32_t focr_hip_qint8_upload(focr_hip_ctx* ctx, const int8_t* w, const float* scales, size_t n,
                               size_t k, focr_hip_qint8** out);
 int32_t focr_hip_qint8_from_device(focr_hip_ctx* ctx, const int8_t* w, const float* scales,
